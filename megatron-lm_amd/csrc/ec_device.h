@@ -132,6 +132,22 @@ __device__ __forceinline__ void store_stream(void* p, const uint4& v) {
   __builtin_nontemporal_store(w, (global_u32x4*)(uintptr_t)p);
 }
 
+// The same at any byte address (a vector type of alignment 1: gfx950 takes
+// the single dwordx4 access, see load_realign).
+typedef uint32_t u32x4_unaligned __attribute__((ext_vector_type(4), aligned(1)));
+typedef __attribute__((address_space(1))) u32x4_unaligned global_u32x4_unaligned;
+
+__device__ __forceinline__ uint4 load_any(const void* p) {
+  const u32x4_unaligned v =
+      __builtin_nontemporal_load((const global_u32x4_unaligned*)(uintptr_t)p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+__device__ __forceinline__ void store_any(void* p, const uint4& v) {
+  const u32x4_unaligned w = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(w, (global_u32x4_unaligned*)(uintptr_t)p);
+}
+
 // The same accesses as buffer instructions on a wave-uniform base: the
 // resource descriptor sits in SGPRs and each lane adds its byte offset
 // (lane_off < 2^31).  The caller guarantees that base is the same for every
@@ -260,8 +276,7 @@ __device__ __forceinline__ void gf_matvec16(uint32_t (&acc)[M][4], const uint4 (
   }
 }
 
-// Device-side field multiply (shift-and-reduce), used only to build the
-// permute tables of the generic kernel in LDS.
+// Device-side field multiply (shift-and-reduce), for shards of a few bytes.
 __device__ inline uint8_t dev_gf_mul(uint32_t a, uint32_t b) {
   uint32_t r = 0;
   for (int i = 0; i < 8; ++i) {
@@ -273,39 +288,40 @@ __device__ inline uint8_t dev_gf_mul(uint32_t a, uint32_t b) {
   return (uint8_t)r;
 }
 
+// The permute tables of coefficient c, for the kernels that build them in LDS.
+// Every entry is an XOR of the products c * 2^b (about 50 VALU ops; a field
+// multiply for each of the 20 entries took over ten times as many).
 __device__ inline PermTab dev_perm_tab(uint32_t c) {
-  PermTab p;
-  uint32_t w[5] = {0, 0, 0, 0, 0};
-  for (int a = 0; a < 8; ++a) {
-    w[a >> 2] |= (uint32_t)dev_gf_mul(c, a) << (8 * (a & 3));
-    w[2 + (a >> 2)] |= (uint32_t)dev_gf_mul(c, a << 3) << (8 * (a & 3));
-  }
-  for (int a = 0; a < 4; ++a) w[4] |= (uint32_t)dev_gf_mul(c, a << 6) << (8 * a);
-  p.lo0 = w[0];
-  p.hi0 = w[1];
-  p.lo1 = w[2];
-  p.hi1 = w[3];
-  p.t2 = w[4];
-  return p;
+  uint32_t p[8];
+  p[0] = c;
+#pragma unroll
+  for (int b = 1; b < 8; ++b) p[b] = (p[b - 1] << 1) ^ (p[b - 1] & 0x80u ? 0x11Du : 0u);
+  const auto quad = [](uint32_t x, uint32_t y) {   // products of 0, 1, 2, 3
+    return (x << 8) | (y << 16) | ((x ^ y) << 24);
+  };
+  PermTab t;
+  t.lo0 = quad(p[0], p[1]);
+  t.hi0 = t.lo0 ^ p[2] * 0x01010101u;
+  t.lo1 = quad(p[3], p[4]);
+  t.hi1 = t.lo1 ^ p[5] * 0x01010101u;
+  t.t2 = quad(p[6], p[7]);
+  return t;
 }
 
 // ------------------------------------------------------- wide-code knobs --
-// Codes past the instantiated fast path (k > 16 or m > 4, up to 32 x 16) on
-// 16-byte-aligned shards: rs_kernel's column layout and launch order with
-// the m outputs in registers (M is a template parameter) and k read at run time
-// in groups of kWideGroup loads in flight.  The m x k tables do not fit the
-// kernel arguments (10 KiB for 16 x 32), so each workgroup builds them in LDS
-// from the coefficient bytes.  Measured over 256 MiB shards (HBM TB/s): a
-// full grid beat grids capped at 4k-32k workgroups (RS(6,8) 5.34 vs
-// 4.5-5.2, RS(24,4) 5.37 vs 4.7-4.9), so the table build costs less than the
-// lost parallelism; groups of 16 loads halved the rate, groups of 4 were
-// 0-15 % slower than 8.
+// The kernels with k at run time on permute tables (table_kernel in
+// ec_flat.hip, batched_wide_kernel and update_wide_kernel in ec_update.hip):
+// the m outputs in registers (M is a template parameter), the shards in groups
+// of kWideGroup loads in flight, the m x k tables built in LDS by each
+// workgroup.  Over 256 MiB shards a full grid beat grids capped at 4k-32k
+// workgroups (RS(6,8) 5.34 vs 4.5-5.2 TB/s of HBM traffic), so the table build
+// costs less than the lost parallelism; groups of 16 loads halved the rate,
+// groups of 4 were 0-15 % slower than 8.
 constexpr int kWideGroup = 8;
 
-// Coefficients per step of the wide kernel's inner loop: pairs for m >= 8,
-// where the GF arithmetic bounds the kernel (RS(32,16) 2.49 -> 2.68 TB/s,
-// RS(10,12) 4.03 -> 4.22), single ones below, where the pair form's longer
-// dependency chains cost 2-6 % (RS(24,4) 5.13 vs 4.90).
+// Coefficients per step of table_kernel's inner loop: pairs for m >= 8, where
+// the GF arithmetic bounds the kernel (RS(10,12) 4.03 -> 4.22 TB/s), single
+// ones below, where the pair form's longer dependency chains cost 2-6 %.
 template <int M>
 constexpr int kWidePair() {
   return M >= 8 ? 2 : 1;
@@ -327,13 +343,9 @@ constexpr int kWidePair() {
 // 4.15, RS(6,3) in 1 MiB units 4.88 -> 5.94 (6.15-6.65 for aligned copies of
 // the same tensors); RS(6,3) over six 64 MiB shards at skews 1-6 through the
 // wide kernel 5.24 -> 5.62.  Aligned inputs do not take this path.
-typedef uint32_t u32x4_unaligned __attribute__((ext_vector_type(4), aligned(1)));
-
 __device__ __forceinline__ uint4 load_realign(const uint8_t* base, uint64_t off) {
   if ((reinterpret_cast<uintptr_t>(base) & 15u) == 0) return load_stream(base + off);
-  const u32x4_unaligned v =
-      __builtin_nontemporal_load(reinterpret_cast<const u32x4_unaligned*>(base + off));
-  return make_uint4(v.x, v.y, v.z, v.w);
+  return load_any(base + off);
 }
 
 // ---------------------------------------------------------- unit access --
@@ -379,22 +391,14 @@ __device__ __forceinline__ void store_unit_len(uint8_t* p, uint32_t off, uint32_
 
 inline int hip_status() { return hipGetLastError() == hipSuccess ? EC_OK : EC_EHIP; }
 
-// Grid for a grid-stride kernel over n16 chunks with U chunks per lane of a
-// kBlock-lane workgroup: enough workgroups to cover the range once, capped so
-// a launch stays a few waves deep on 256 CUs.
-inline unsigned grid_for(uint64_t n16, int U) {
-  const uint64_t tiles = (n16 + (uint64_t)kBlock * U - 1) / ((uint64_t)kBlock * U);
-  const uint64_t cap = 1u << 20;
-  return (unsigned)(tiles < cap ? (tiles ? tiles : 1) : cap);
-}
+constexpr uint64_t kMaxGrid = 1u << 24;   // workgroups of a flat launch; more work loops
 
 // Grid of a grid-stride kernel with `lanes` lanes per workgroup and one chunk
 // per lane: one workgroup per `lanes` chunks, up to 2^24 workgroups (shards
 // up to 16 GiB with 64 lanes are covered in one pass).
 inline unsigned grid_of(uint64_t n16, int lanes) {
   const uint64_t g = (n16 + (uint64_t)lanes - 1) / (uint64_t)lanes;
-  const uint64_t cap = 1u << 24;
-  return (unsigned)(g < cap ? (g ? g : 1) : cap);
+  return (unsigned)(g < kMaxGrid ? (g ? g : 1) : kMaxGrid);
 }
 
 // ----------------------------------------- grid order of batched launches --

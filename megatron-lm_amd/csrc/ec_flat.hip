@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "ec_device.h"
+#include "ec_mfma.h"
 
 namespace ec {
 namespace {
@@ -186,45 +187,165 @@ __global__ void __launch_bounds__(kXorBlock) xor_kernel(const XorArgs<K> a) {
   }
 }
 
-// --------------------------------------------------------- generic kernel --
-// Any k <= EC_MAX_K, m <= EC_MAX_M and any alignment: byte loads and stores,
-// four bytes per lane, permute tables built in LDS by the workgroup.  Used for
-// shard counts beyond the instantiated ones, misaligned pointers and the
-// sub-16-byte tail of the fast kernels.
-
-struct GenArgs {
-  const uint8_t* data[EC_MAX_K];
-  uint8_t* out[EC_MAX_M];
-  uint8_t coeff[EC_MAX_M * EC_MAX_K];
-  uint64_t n;
-  int k, m;
+// ------------------------------------------------------------- any shards --
+// Shards of any byte size (16 and more) at any alignment, in one launch: a
+// frame of 16-byte chunks that starts `head` bytes into the shards (so that
+// the outputs, or most of them, are aligned there) goes through the vector
+// code with unaligned accesses.  The up to 15 bytes before and after it are
+// the first and the last bytes of one more 16-byte chunk each, at the shards'
+// start and at their end: it is loaded and coded whole, and only its own
+// bytes are stored, one by one (the others belong to the frame).  Whole chunks
+// at aligned addresses keep rs_kernel and xor_kernel.
+struct Frame {
+  uint64_t nbytes;  // of a shard
+  uint64_t n16;     // chunks
+  uint32_t head;    // bytes before them
+  uint32_t tail;    // bytes after them
 };
 
-__global__ void __launch_bounds__(kBlock) generic_kernel(const GenArgs a) {
-  __shared__ PermTab tab[EC_MAX_M * EC_MAX_K];
-  for (int t = threadIdx.x; t < a.m * a.k; t += kBlock) tab[t] = dev_perm_tab(a.coeff[t]);
-  __syncthreads();
-  const uint64_t n4 = (a.n + 3) / 4;
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-  for (uint64_t q = (uint64_t)blockIdx.x * kBlock + threadIdx.x; q < n4; q += stride) {
-    const uint64_t b0 = q * 4;
-    const int nb = (int)((a.n - b0) < 4 ? (a.n - b0) : 4);
-    uint32_t acc[EC_MAX_M];
-    for (int i = 0; i < a.m; ++i) acc[i] = 0;
-    for (int j = 0; j < a.k; ++j) {
-      uint32_t w = 0;
-      for (int b = 0; b < nb; ++b) w |= (uint32_t)a.data[j][b0 + b] << (8 * b);
-      const Fields f = fields(w);
-      for (int i = 0; i < a.m; ++i) acc[i] = mac1(acc[i], tab[i * a.k + j], f);
-    }
-    for (int i = 0; i < a.m; ++i)
-      for (int b = 0; b < nb; ++b) a.out[i][b0 + b] = (uint8_t)(acc[i] >> (8 * b));
+// A step of the launch: 0 and 1 the head and the tail where there are any,
+// then the frame's.  Everything here is uniform over the workgroup (or wave).
+struct Step {
+  uint64_t at;         // byte offset of the step's first chunk
+  uint64_t chunks;     // chunks from there to the frame's end (an edge: 1)
+  uint32_t from, to;   // bytes of the chunk to store: 0, 16 except at an edge
+};
+
+__device__ __forceinline__ uint32_t edge_steps(const Frame& f) {
+  return (f.head != 0) + (f.tail != 0);
+}
+
+__device__ __forceinline__ Step step_of(const Frame& f, uint64_t step, uint32_t chunks_per_step) {
+  const uint32_t edges = edge_steps(f);
+  if (step >= edges) {
+    const uint64_t first = (step - edges) * chunks_per_step;
+    return {f.head + first * 16, f.n16 - first, 0u, 16u};
+  }
+  if (f.head != 0 && step == 0) return {0, 1, 0u, f.head};
+  return {f.nbytes - 16, 1, 16u - f.tail, 16u};
+}
+
+__device__ __forceinline__ bool whole(const Step& s) { return s.to - s.from == 16u; }
+
+// Bytes [from, to) of v, one at a time.
+__device__ __forceinline__ void store_edge(uint8_t* p, const Step& s, uint4 v) {
+#pragma unroll 1
+  for (uint32_t b = 0; b < s.to; ++b) {   // shifted down, so that no register is indexed
+    if (b >= s.from) gptr(p)[b] = (uint8_t)v.x;
+    v = make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, 1), __builtin_amdgcn_alignbyte(v.z, v.y, 1),
+                   __builtin_amdgcn_alignbyte(v.w, v.z, 1), v.w >> 8);
   }
 }
 
-// ------------------------------------------------------------ wide kernel --
-// Codes past the instantiated fast path: see kWideGroup in ec_device.h.
-struct WideArgs {
+template <int M>
+__device__ __forceinline__ void store_outputs(uint8_t* const (&out)[M], uint64_t off, const Step& s,
+                                              const uint32_t (&acc)[M][4]) {
+  if (whole(s)) {
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      store_any(out[i] + off, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
+  } else {
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      store_edge(out[i] + off, s, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
+  }
+}
+
+// All products here, not each output's sunk into the branches of its store
+// (RS(12,4) in any_kernel: the tables would stay live in 340 registers).
+template <int M>
+__device__ __forceinline__ void pin_products(uint32_t (&acc)[M][4]) {
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+#pragma unroll
+    for (int dd = 0; dd < 4; ++dd) asm volatile("" : "+v"(acc[i][dd]));
+}
+
+template <int K, int M>
+struct AnyArgs {
+  const uint8_t* data[K];
+  uint8_t* out[M];
+  PermTab tab[M][K];
+  Frame f;
+};
+
+template <int K, int M, bool PASSES>
+__global__ void __launch_bounds__((flat_block<K, M>())) any_kernel(const AnyArgs<K, M> a) {
+  constexpr int B = flat_block<K, M>();
+  __shared__ PermTab tab[M][K];
+  for (int q = threadIdx.x; q < M * K; q += B) tab[q / K][q % K] = a.tab[q / K][q % K];
+  __syncthreads();
+  const uint64_t steps = PASSES ? edge_steps(a.f) + (a.f.n16 + B - 1) / B : 0;
+  for (uint64_t step = blockIdx.x;;) {
+    const Step s = step_of(a.f, step, B);
+    if (threadIdx.x < s.chunks) {
+      const uint32_t lane = threadIdx.x * 16u;
+      uint4 x[K];
+#pragma unroll
+      for (int j = 0; j < K; ++j) x[j] = load_any(a.data[j] + s.at + lane);
+      uint32_t acc[M][4] = {};
+      gf_matvec16<K, M>(acc, x, tab);
+      pin_products(acc);
+      store_outputs(a.out, s.at + lane, s, acc);
+    }
+    step += gridDim.x;
+    if (!PASSES || step >= steps) break;
+  }
+}
+
+template <int K>
+struct AnyXorArgs {
+  const uint8_t* data[K];
+  uint8_t* out;
+  Frame f;
+};
+
+template <int K>
+__global__ void __launch_bounds__(kXorBlock) any_xor_kernel(const AnyXorArgs<K> a) {
+  const uint64_t steps = edge_steps(a.f) + (a.f.n16 + kXorBlock - 1) / kXorBlock;
+  for (uint64_t step = blockIdx.x; step < steps; step += gridDim.x) {
+    const Step s = step_of(a.f, step, kXorBlock);
+    if (threadIdx.x >= s.chunks) continue;
+    const uint32_t lane = threadIdx.x * 16u;
+    uint4 x[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) x[j] = load_any(a.data[j] + s.at + lane);
+    uint4 acc = x[0];
+    int j = 1;
+#pragma unroll
+    for (; j + 1 < K; j += 2) acc = xor3v(acc, x[j], x[j + 1]);
+    if (j < K) acc = make_uint4(acc.x ^ x[j].x, acc.y ^ x[j].y, acc.z ^ x[j].z, acc.w ^ x[j].w);
+    if (whole(s))
+      store_any(a.out + s.at + lane, acc);
+    else
+      store_edge(a.out + s.at + lane, s, acc);
+  }
+}
+
+// Shards of less than 16 bytes: one lane per byte, any k and m.
+struct TinyArgs {
+  const uint8_t* data[EC_MAX_K];
+  uint8_t* out[EC_MAX_M];
+  uint8_t coeff[EC_MAX_M * EC_MAX_K];
+  uint32_t n;
+  int k, m;
+};
+
+__global__ void __launch_bounds__(64) tiny_kernel(const TinyArgs a) {
+  const uint32_t b = threadIdx.x & 15u;
+  if (b >= a.n) return;
+  for (int i = threadIdx.x >> 4; i < a.m; i += 4) {
+    uint8_t acc = 0;
+    for (int j = 0; j < a.k; ++j) acc ^= dev_gf_mul(a.coeff[i * a.k + j], gptr(a.data[j])[b]);
+    gptr(a.out[i])[b] = acc;
+  }
+}
+
+// ------------------------------------------------------------ table kernel --
+// Codes past the unrolled kernels for which the permute tables cost less than
+// the matrix cores (see matvec), on whole chunks at aligned addresses: see
+// kWideGroup in ec_device.h.
+struct TableArgs {
   const uint8_t* data[EC_MAX_K];
   uint8_t* out[EC_MAX_M];
   uint8_t coeff[EC_MAX_M * EC_MAX_K];  // row-major m x k
@@ -233,20 +354,19 @@ struct WideArgs {
 };
 
 // 128-lane workgroups in launch order.  Measured on MI355X (HBM traffic,
-// GB/s; the former 256-lane workgroups that streamed each shard at two
-// places half a shard apart first): RS(20,4) over 256 MiB 5157 -> 5464, RS(24,4) 5124 ->
-// 5385, RS(10,6) over 128 MiB 5280 -> 5311, RS(6,8) 4844 -> 4902, RS(32,16)
-// over 64 MiB 2720 -> 2700 (VALU-bound there).
-constexpr int kWideBlock = 128;
+// TB/s, 64 MiB shards): RS(17,1) 6.1, RS(20,2) 5.8, RS(6,12) 5.5, RS(10,12)
+// 4.6; 256-lane workgroups that streamed each shard at two places half a shard
+// apart were 1-6 % slower.
+constexpr int kTableBlock = 128;
 
 template <int M>
-__global__ void __launch_bounds__(kWideBlock) wide_kernel(const WideArgs a) {
+__global__ void __launch_bounds__(kTableBlock) table_kernel(const TableArgs a) {
   __shared__ PermTab tab[M * EC_MAX_K];
   const int k = a.k;
-  for (int t = threadIdx.x; t < M * k; t += kWideBlock) tab[t] = dev_perm_tab(a.coeff[t]);
+  for (int t = threadIdx.x; t < M * k; t += kTableBlock) tab[t] = dev_perm_tab(a.coeff[t]);
   __syncthreads();
-  const uint64_t stride = (uint64_t)gridDim.x * kWideBlock;
-  for (uint64_t idx = (uint64_t)blockIdx.x * kWideBlock + threadIdx.x;
+  const uint64_t stride = (uint64_t)gridDim.x * kTableBlock;
+  for (uint64_t idx = (uint64_t)blockIdx.x * kTableBlock + threadIdx.x;
        idx < a.n16; idx += stride) {
     uint32_t acc[M][4] = {};
     for (int j0 = 0; j0 < k; j0 += kWideGroup) {
@@ -296,6 +416,172 @@ __global__ void __launch_bounds__(kWideBlock) wide_kernel(const WideArgs a) {
   }
 }
 
+// ------------------------------------------------------------ wide kernels --
+// Codes past the unrolled kernels, any alignment and size, on the matrix cores
+// (ec_mfma.h).  A wave codes 32 chunks (512 bytes of each shard) per step:
+// lane l and lane l + 32 load the same columns of the even and the odd shards,
+// and store those of the even and the odd outputs.
+//   m > 4 (wide_kernel): the MFMAs and bit selects take about as long as the
+// memory traffic, so waves stay and load their next step while they code one.
+// Measured on MI355X (HBM traffic, TB/s; the former run-time-k kernel on
+// permute tables first): RS(24,8) over 32 MiB shards 4.08 -> 5.38 (one step
+// per wave without the loads ahead 5.19), RS(32,16) 2.69 -> 3.93 (3.10),
+// RS(20,12) 3.57 -> 4.27 (3.80), RS(16,8) over 64 MiB 4.47 -> 5.61 (5.16).
+// With the MFMAs taken out the same kernel moves 5.7-6.0.
+//   m <= 4 (wide_narrow_kernel): memory-bound, one step per wave and none
+// ahead: RS(20,4) over 64 MiB 5.70 -> 6.12 (with loads ahead 5.6), RS(24,4)
+// 5.62 -> 5.90.
+struct WideArgs {
+  const uint8_t* data[EC_MAX_K];   // data[k] = data[k - 1] when k is odd
+  uint8_t* out[EC_MAX_M];
+  MfmaCoeff coeff;
+  Frame f;
+  int k, m;
+};
+
+// even or odd by the lane's half.  Both are read into scalar registers first:
+// the compiler would otherwise select the address to read them from, one
+// dependent vector load each.
+template <typename T>
+__device__ __forceinline__ T* of_half(uint32_t half, T* even, T* odd) {
+  asm volatile("" : "+s"(even), "+s"(odd));
+  return half ? odd : even;
+}
+
+constexpr int kWideBlock = 256;
+constexpr int kWideChunks = 32;   // chunks of a wave's step
+
+template <int KH, int MH>
+struct WideLds {
+  const uint8_t* data[EC_MAX_K];
+  uint8_t* out[EC_MAX_M];
+  typename MfmaCode<KH, MH>::Lds code;
+};
+
+// The loads of a step: x[kt][i] of shard 8 kt + 2 i + h, 16 bytes at off.
+template <int KH>
+__device__ __forceinline__ void wide_loads(uint4 (&x)[mfma_groups(KH)][4],
+                                           const uint8_t* const* data, int k, uint32_t half,
+                                           uint64_t off) {
+#pragma unroll
+  for (int kt = 0; kt < mfma_groups(KH); ++kt)
+#pragma unroll
+    for (int i = 0; i < mfma_words(KH, kt); ++i) {
+      const int even = 8 * kt + 2 * i;
+      if (even < 4 * KH - 3 || even < k)   // uniform: the first always, k > 4 (KH - 1)
+        x[kt][i] = load_any(data[even + half] + off);
+      else
+        x[kt][i] = make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+
+template <int KH, int MH, bool PAIR>
+__global__ void __launch_bounds__(kWideBlock) __attribute__((amdgpu_waves_per_eu(2)))
+wide_kernel(const WideArgs a) {
+  constexpr int KT = mfma_groups(KH), MT = mfma_tiles(MH);
+  __shared__ WideLds<KH, MH> lds;
+  if (threadIdx.x < EC_MAX_K) lds.data[threadIdx.x] = a.data[threadIdx.x];
+  else if (threadIdx.x < EC_MAX_K + EC_MAX_M)
+    lds.out[threadIdx.x - EC_MAX_K] = a.out[threadIdx.x - EC_MAX_K];
+  MfmaCode<KH, MH> code;
+  code.template load<kWideBlock>(a.coeff, lds.code);
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63u, col = lane & 31u, half = lane >> 5;
+  const uint64_t steps = edge_steps(a.f) + (a.f.n16 + kWideChunks - 1) / kWideChunks;
+  const uint64_t stride = (uint64_t)gridDim.x * (kWideBlock / 64);
+  uint64_t step = (uint64_t)blockIdx.x * (kWideBlock / 64) +
+                  __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (step >= steps) return;
+  Step s = step_of(a.f, step, kWideChunks);
+  uint64_t off = s.at + (col < s.chunks ? col * 16u : 0u);   // past the end: the first chunk
+  uint4 x[KT][4];
+  wide_loads<KH>(x, lds.data, a.k, half, off);
+  for (;;) {
+    uint32_t t[KT][4][4];
+    mfma_columns<KH, true>(t, x);
+    // The next step's loads are in flight while this one is coded.
+    const Step now = s;
+    const uint64_t at = off;
+    const bool mine = col < now.chunks;
+    step += stride;
+    const bool more = step < steps;   // uniform
+    asm volatile("" ::: "memory");    // the addresses stay in LDS
+    if (more) {
+      s = step_of(a.f, step, kWideChunks);
+      off = s.at + (col < s.chunks ? col * 16u : 0u);
+      wide_loads<KH>(x, lds.data, a.k, half, off);
+    }
+    uint4 out[MT][2];
+    mfma_matvec16<KH, MH, PAIR>(out, t, code);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int q = 0; q < mfma_outs(MH, mt); ++q) {
+        const uint32_t o = 4 * mt + 2 * q + half;
+        if (!mine || (int)o >= a.m) continue;
+        if (whole(now))
+          store_any(lds.out[o] + at, out[mt][q]);
+        else
+          store_edge(lds.out[o] + at, now, out[mt][q]);
+      }
+    if (!more) break;
+  }
+}
+
+template <int KH, int MH, bool PAIR>
+__global__ void __launch_bounds__(kWideBlock)
+__attribute__((amdgpu_waves_per_eu(2))) wide_narrow_kernel(const WideArgs a) {
+  constexpr int KT = mfma_groups(KH);
+  static_assert(mfma_tiles(MH) == 1 && !MfmaCode<KH, MH>::kInLds, "m <= 4");
+  const uint32_t lane = threadIdx.x & 63u, col = lane & 31u, half = lane >> 5;
+  const uint64_t steps = edge_steps(a.f) + (a.f.n16 + kWideChunks - 1) / kWideChunks;
+  const uint64_t stride = (uint64_t)gridDim.x * (kWideBlock / 64);
+  uint64_t step = (uint64_t)blockIdx.x * (kWideBlock / 64) +
+                  __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (step >= steps) return;
+  const uint8_t* data[KT][4];
+  uint8_t* outp[2];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < mfma_words(KH, kt); ++i)
+      data[kt][i] = of_half(half, a.data[8 * kt + 2 * i], a.data[8 * kt + 2 * i + 1]);
+#pragma unroll
+  for (int q = 0; q < mfma_outs(MH, 0); ++q) outp[q] = of_half(half, a.out[2 * q], a.out[2 * q + 1]);
+  __shared__ typename MfmaCode<KH, MH>::Lds unused;
+  MfmaCode<KH, MH> code;
+  code.template load<kWideBlock>(a.coeff, unused);
+  for (; step < steps; step += stride) {
+    const Step s = step_of(a.f, step, kWideChunks);
+    const bool mine = col < s.chunks;
+    const uint64_t off = s.at + (mine ? col * 16u : 0u);   // past the end: the first chunk
+    uint4 x[KT][4];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < mfma_words(KH, kt); ++i) {
+        const int even = 8 * kt + 2 * i;
+        if (even < 4 * KH - 3 || even < a.k)   // uniform, as in wide_loads
+          x[kt][i] = load_any(data[kt][i] + off);
+        else
+          x[kt][i] = make_uint4(0u, 0u, 0u, 0u);
+      }
+    uint32_t t[KT][4][4];
+    mfma_columns<KH, false>(t, x);
+    uint4 out[1][2];
+    mfma_matvec16<KH, MH, PAIR>(out, t, code);
+#pragma unroll
+    for (int q = 0; q < mfma_outs(MH, 0); ++q) {
+      if (!mine || (int)(2 * q + half) >= a.m) continue;
+      if (whole(s))
+        store_any(outp[q] + off, out[0][q]);
+      else
+        store_edge(outp[q] + off, s, out[0][q]);
+    }
+  }
+}
+
 // ---------------------------------------------------------- host launch --
 
 template <int K, int M>
@@ -321,16 +607,96 @@ int launch_rs(const uint8_t* coeff, const uint8_t* const* d, uint8_t* const* o, 
   return hip_status();
 }
 
-template <int M>
-int launch_wide(const uint8_t* coeff, int k, const uint8_t* const* d, uint8_t* const* o,
-                uint64_t n16, hipStream_t st) {
+using WideFn = int (*)(const uint8_t*, int, int, const uint8_t* const*, uint8_t* const*,
+                       const Frame&, hipStream_t);
+WideFn wide_fn(int k, int m);
+
+inline uint64_t frame_steps(const Frame& f, uint64_t chunks_per_step) {
+  return (f.head != 0) + (f.tail != 0) + (f.n16 + chunks_per_step - 1) / chunks_per_step;
+}
+
+template <int K, int M>
+int launch_any(const uint8_t* coeff, const uint8_t* const* d, uint8_t* const* o, const Frame& f,
+               hipStream_t st) {
+  AnyArgs<K, M> a;
+  for (int j = 0; j < K; ++j) a.data[j] = d[j];
+  for (int i = 0; i < M; ++i) a.out[i] = o[i];
+  for (int i = 0; i < M; ++i)
+    for (int j = 0; j < K; ++j) a.tab[i][j] = perm_tab(coeff[i * K + j]);
+  a.f = f;
+  constexpr int B = flat_block<K, M>();
+  const uint64_t steps = frame_steps(f, B);
+  const unsigned grid = (unsigned)(steps < kMaxGrid ? steps : kMaxGrid);
+  if (grid == steps)
+    hipLaunchKernelGGL((any_kernel<K, M, false>), dim3(grid), dim3(B), 0, st, a);
+  else if constexpr (M <= kFastMaxM)
+    hipLaunchKernelGGL((any_kernel<K, M, true>), dim3(grid), dim3(B), 0, st, a);
+  else   // shards past 32 GiB
+    return wide_fn(K, M)(coeff, K, M, d, o, f, st);
+  return hip_status();
+}
+
+template <int K>
+int launch_any_xor(const uint8_t* const* d, uint8_t* o, const Frame& f, hipStream_t st) {
+  AnyXorArgs<K> a;
+  for (int j = 0; j < K; ++j) a.data[j] = d[j];
+  a.out = o;
+  a.f = f;
+  const uint64_t steps = frame_steps(f, kXorBlock);
+  hipLaunchKernelGGL((any_xor_kernel<K>), dim3((unsigned)(steps < kMaxGrid ? steps : kMaxGrid)),
+                     dim3(kXorBlock), 0, st, a);
+  return hip_status();
+}
+
+// Workgroups of a wide_kernel launch.  About one for each that the chip holds
+// for the deep codes (2 waves per SIMD), several where more waves fit: capped
+// at 1024 / 4096, RS(24,8) over 32 MiB 199.7 / 209.3 us, RS(32,16) 410 / 420,
+// RS(20,12) 251 / 261, but RS(16,8) over 64 MiB 294.7 / 287.2, RS(16,6) 267 / 263.
+constexpr uint64_t kWideGridDeep = 1024, kWideGrid = 4096;
+
+template <int KH, int MH>
+int launch_wide(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uint8_t* const* o,
+                const Frame& f, hipStream_t st) {
   WideArgs a;
+  // With k odd the upper lanes read the last shard as well (their
+  // coefficients for it are zero).
+  for (int j = 0; j < EC_MAX_K; ++j) a.data[j] = j < k ? d[j] : j == k ? d[k - 1] : nullptr;
+  for (int i = 0; i < EC_MAX_M; ++i) a.out[i] = i < m ? o[i] : nullptr;
+  a.coeff = mfma_coeff(coeff, k, m);
+  a.f = f;
+  a.k = k;
+  a.m = m;
+  constexpr uint64_t kWaves = kWideBlock / 64;
+  const uint64_t blocks = (frame_steps(f, kWideChunks) + kWaves - 1) / kWaves;
+  const uint64_t cap = MH <= 2 ? kMaxGrid : mfma_groups(KH) >= 3 ? kWideGridDeep : kWideGrid;
+  const dim3 grid((unsigned)(blocks < cap ? blocks : cap)), block(kWideBlock);
+  bool pair = true;
+  if constexpr (KH == EC_MAX_K / 4) pair = mfma_pair_ok(coeff, k, m);
+  if constexpr (MH <= 2) {
+    if (pair)
+      hipLaunchKernelGGL((wide_narrow_kernel<KH, MH, true>), grid, block, 0, st, a);
+    else if constexpr (KH == EC_MAX_K / 4)
+      hipLaunchKernelGGL((wide_narrow_kernel<KH, MH, false>), grid, block, 0, st, a);
+  } else {
+    if (pair)
+      hipLaunchKernelGGL((wide_kernel<KH, MH, true>), grid, block, 0, st, a);
+    else if constexpr (KH == EC_MAX_K / 4)
+      hipLaunchKernelGGL((wide_kernel<KH, MH, false>), grid, block, 0, st, a);
+  }
+  return hip_status();
+}
+
+template <int M>
+int launch_table(const uint8_t* coeff, int k, const uint8_t* const* d, uint8_t* const* o,
+                 uint64_t n16, hipStream_t st) {
+  TableArgs a;
   for (int j = 0; j < k; ++j) a.data[j] = d[j];
   for (int i = 0; i < M; ++i) a.out[i] = o[i];
   for (int t = 0; t < M * k; ++t) a.coeff[t] = coeff[t];
   a.n16 = n16;
   a.k = k;
-  hipLaunchKernelGGL((wide_kernel<M>), dim3(grid_of(n16, kWideBlock)), dim3(kWideBlock), 0, st, a);
+  hipLaunchKernelGGL((table_kernel<M>), dim3(grid_of(n16, kTableBlock)), dim3(kTableBlock), 0, st,
+                     a);
   return hip_status();
 }
 
@@ -351,6 +717,9 @@ int launch_xor(const uint8_t* const* d, uint8_t* o, uint64_t n16, hipStream_t st
 using RsFn = int (*)(const uint8_t*, const uint8_t* const*, uint8_t* const*, uint64_t,
                      hipStream_t);
 using XorFn = int (*)(const uint8_t* const*, uint8_t*, uint64_t, hipStream_t);
+using AnyFn = int (*)(const uint8_t*, const uint8_t* const*, uint8_t* const*, const Frame&,
+                      hipStream_t);
+using AnyXorFn = int (*)(const uint8_t* const*, uint8_t*, const Frame&, hipStream_t);
 
 template <int K, int... Ms>
 constexpr auto rs_row(std::integer_sequence<int, Ms...>) {
@@ -365,42 +734,119 @@ template <int... Ks>
 constexpr auto xor_table(std::integer_sequence<int, Ks...>) {
   return std::array<XorFn, sizeof...(Ks)>{&launch_xor<Ks + 1>...};
 }
-using WideFn = int (*)(const uint8_t*, int, const uint8_t* const*, uint8_t* const*, uint64_t,
-                       hipStream_t);
+template <int K, int... Ms>
+constexpr auto any_row(std::integer_sequence<int, Ms...>) {
+  return std::array<AnyFn, sizeof...(Ms)>{&launch_any<K, Ms + 1>...};
+}
+constexpr int kAnyMaxM = 8, kAnyDeepMaxK = 12;   // M > kFastMaxM: k <= kAnyDeepMaxK
+template <int K>
+constexpr auto any_row_of() {
+  constexpr int kMs = K <= kAnyDeepMaxK ? kAnyMaxM : kFastMaxM;
+  std::array<AnyFn, kAnyMaxM> r{};
+  const auto row = any_row<K>(std::make_integer_sequence<int, kMs>{});
+  for (int i = 0; i < kMs; ++i) r[i] = row[i];
+  return r;
+}
+template <int... Ks>
+constexpr auto any_table(std::integer_sequence<int, Ks...>) {
+  return std::array<std::array<AnyFn, kAnyMaxM>, sizeof...(Ks)>{any_row_of<Ks + 1>()...};
+}
+template <int... Ks>
+constexpr auto any_xor_table(std::integer_sequence<int, Ks...>) {
+  return std::array<AnyXorFn, sizeof...(Ks)>{&launch_any_xor<Ks + 1>...};
+}
+using TableFn = int (*)(const uint8_t*, int, const uint8_t* const*, uint8_t* const*, uint64_t,
+                        hipStream_t);
 template <int... Ms>
-constexpr auto wide_table(std::integer_sequence<int, Ms...>) {
-  return std::array<WideFn, sizeof...(Ms)>{&launch_wide<Ms + 1>...};
+constexpr auto table_table(std::integer_sequence<int, Ms...>) {
+  return std::array<TableFn, sizeof...(Ms)>{&launch_table<Ms + 1>...};
+}
+template <int KH, int... Ms>
+constexpr auto wide_row(std::integer_sequence<int, Ms...>) {
+  return std::array<WideFn, sizeof...(Ms)>{&launch_wide<KH, Ms + 1>...};
+}
+constexpr int kWideKH = EC_MAX_K / 4, kWideMH = EC_MAX_M / 2;
+template <int... Ks>
+constexpr auto wide_table(std::integer_sequence<int, Ks...>) {
+  return std::array<std::array<WideFn, kWideMH>, sizeof...(Ks)>{
+      wide_row<Ks + 1>(std::make_integer_sequence<int, kWideMH>{})...};
 }
 
 const auto kRsTable = rs_table(std::make_integer_sequence<int, kFastMaxK>{});
 const auto kXorTable = xor_table(std::make_integer_sequence<int, kFastMaxK>{});
-const auto kWideTable = wide_table(std::make_integer_sequence<int, EC_MAX_M>{});
+const auto kAnyTable = any_table(std::make_integer_sequence<int, kFastMaxK>{});
+const auto kAnyXorTable = any_xor_table(std::make_integer_sequence<int, kFastMaxK>{});
+const auto kTableTable = table_table(std::make_integer_sequence<int, EC_MAX_M>{});
+const auto kWideTable = wide_table(std::make_integer_sequence<int, kWideKH>{});
 
-int launch_generic(const uint8_t* coeff, int k, int m, const uint8_t* const* d,
-                   uint8_t* const* o, uint64_t offset, uint64_t n, hipStream_t st) {
-  GenArgs a;
-  for (int j = 0; j < k; ++j) a.data[j] = d[j] + offset;
-  for (int i = 0; i < m; ++i) a.out[i] = o[i] + offset;
-  for (int t = 0; t < m * k; ++t) a.coeff[t] = coeff[t];
-  a.n = n;
-  a.k = k;
-  a.m = m;
-  const uint64_t n4 = (n + 3) / 4;
-  uint64_t blocks = (n4 + kBlock - 1) / kBlock;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(generic_kernel, dim3((unsigned)(blocks ? blocks : 1)), dim3(kBlock), 0, st,
-                     a);
-  return hip_status();
+WideFn wide_fn(int k, int m) {
+  return kWideTable[(k - 1) / 4][(m - 1) / 2];
 }
 
-// Common misalignment of a set of addresses modulo 16, or -1 if they differ.
-inline int common_skew(const uint8_t* const* a, int n, int skew) {
-  for (int i = 0; i < n; ++i) {
-    const int s = (int)(reinterpret_cast<uintptr_t>(a[i]) & 15u);
-    if (skew < 0) skew = s;
-    else if (s != skew) return -1;
-  }
-  return skew;
+// The address modulo 16 that most of n addresses share.
+inline uint32_t usual_skew(uint8_t* const* a, int n) {
+  int count[16] = {};
+  for (int i = 0; i < n; ++i) ++count[reinterpret_cast<uintptr_t>(a[i]) & 15u];
+  uint32_t best = 0;
+  for (uint32_t s = 1; s < 16; ++s)
+    if (count[s] > count[best]) best = s;
+  return best;
+}
+
+inline bool all_aligned(const uint8_t* const* a, int n) {
+  uintptr_t bits = 0;
+  for (int i = 0; i < n; ++i) bits |= reinterpret_cast<uintptr_t>(a[i]);
+  return (bits & 15u) == 0;
+}
+
+// The frame of nbytes-long shards with outputs o: its chunks start where most
+// outputs are 16-byte aligned.
+inline Frame frame_of(uint8_t* const* o, int m, uint64_t nbytes) {
+  Frame f;
+  f.nbytes = nbytes;
+  const uint32_t skew = usual_skew(o, m);
+  f.head = skew ? 16u - skew : 0u;
+  if (f.head > nbytes) f.head = (uint32_t)nbytes;
+  f.n16 = (nbytes - f.head) / 16;
+  f.tail = (uint32_t)(nbytes - f.head - f.n16 * 16);
+  return f;
+}
+
+// Whether the permute tables take fewer cycles than the matrix cores for a
+// code past the unrolled kernels: SIMD cycles per 512 byte columns, 4 per VALU
+// op (1.125 k m + 1.25 k ops per column against the transposes, expansions and
+// bit selects of ec_mfma.h) and 32 per MFMA; the two kinds measured as good as
+// additive.  Both kernels over 64 MiB shards (HBM traffic, TB/s, tables /
+// matrix cores; * any_kernel's tables): RS(17,1) 6.03 / 5.48, RS(6,9) 5.59 /
+// 4.91, RS(4,16) 5.43 / 4.75, RS(10,10) 4.73 / 4.07, RS(20,5) 5.14 / 4.82,
+// RS(10,6) 5.95* / 4.82, RS(5,5) 5.92* / 5.02, RS(12,8) 5.17* / 5.24, and past
+// the line RS(8,12) 4.92 / 5.40, RS(16,6) 4.87 / 5.55, RS(20,4) 5.60 / 6.04,
+// RS(16,8) 4.36 / 5.55, RS(24,8) 4.09 / 5.38, RS(32,16) 2.69 / 3.93.
+bool table_pays(int k, int m) {
+  const int kt = (k + kMfmaShards - 1) / kMfmaShards, mt = (m + kMfmaOutputs - 1) / kMfmaOutputs;
+  const int tables = 36 * k * m + 40 * k;
+  const int cores = 512 * kt * mt + 448 * kt + 240 * ((m + 1) / 2);
+  return tables <= cores;
+}
+
+// Up to this shard size too few waves run to be bound by either's arithmetic
+// and the matrix cores' shorter chains win for every code (2 MiB shards, us,
+// tables / matrix cores: RS(20,2) 11.9 / 10.7, RS(6,12) 11.3 / 10.5, RS(17,1)
+// 9.9 / 9.6, RS(16,5) 14.1 / 12.2; 4 MiB: 19.1 / 21.3, 18.4 / 20.7, 17.0 /
+// 19.5, 22.6 / 23.3).
+constexpr uint64_t kTableMinBytes = 2u << 20;
+
+int launch_tiny(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uint8_t* const* o,
+                uint64_t n, hipStream_t st) {
+  TinyArgs a;
+  for (int j = 0; j < k; ++j) a.data[j] = d[j];
+  for (int i = 0; i < m; ++i) a.out[i] = o[i];
+  for (int t = 0; t < m * k; ++t) a.coeff[t] = coeff[t];
+  a.n = (uint32_t)n;
+  a.k = k;
+  a.m = m;
+  hipLaunchKernelGGL(tiny_kernel, dim3(1), dim3(64), 0, st, a);
+  return hip_status();
 }
 
 int matvec(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uint8_t* const* o,
@@ -413,33 +859,19 @@ int matvec(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uint8_t*
     if (!d[j]) return EC_EINVAL;
   for (int i = 0; i < m; ++i)
     if (!o[i]) return EC_EINVAL;
-  // The outputs fix the frame: the bytes up to their next 16-byte boundary
-  // run through the byte kernel, the 16-byte columns after it through a
-  // vector kernel (the fast one when every input shares the outputs'
-  // misalignment, else the wide one, which realigns each input), and the
-  // last partial column through the byte kernel.  Outputs of different
-  // misalignments take the byte kernel throughout.
-  const int skew = common_skew(o, m, -1);
-  if (skew < 0) return launch_generic(coeff, k, m, d, o, 0, nbytes, st);
-  const bool same = common_skew(d, k, skew) == skew;
-  uint64_t head = skew ? 16u - (uint64_t)skew : 0;
-  if (head > nbytes) head = nbytes;
-  int s = EC_OK;
-  if (head) s = launch_generic(coeff, k, m, d, o, 0, head, st);
-  const uint64_t n16 = (nbytes - head) / 16;
-  if (s == EC_OK && n16) {
-    const uint8_t* da[EC_MAX_K];
-    uint8_t* oa[EC_MAX_M];
-    for (int j = 0; j < k; ++j) da[j] = d[j] + head;
-    for (int i = 0; i < m; ++i) oa[i] = o[i] + head;
-    if (same && k <= kFastMaxK && m <= kFastMaxM)
-      s = kRsTable[k - 1][m - 1](coeff, da, oa, n16, st);
-    else
-      s = kWideTable[m - 1](coeff, k, da, oa, n16, st);
+  if (nbytes < 16) return launch_tiny(coeff, k, m, d, o, nbytes, st);
+  if (fast_shape(k, m)) {
+    if (nbytes % 16 == 0 && all_aligned(d, k) && all_aligned(o, m))
+      return kRsTable[k - 1][m - 1](coeff, d, o, nbytes / 16, st);
+    return kAnyTable[k - 1][m - 1](coeff, d, o, frame_of(o, m, nbytes), st);
   }
-  const uint64_t done = head + n16 * 16;
-  if (s == EC_OK && done < nbytes) s = launch_generic(coeff, k, m, d, o, done, nbytes - done, st);
-  return s;
+  if (nbytes > kTableMinBytes && table_pays(k, m)) {
+    if (m <= kAnyMaxM && k <= kAnyDeepMaxK)
+      return kAnyTable[k - 1][m - 1](coeff, d, o, frame_of(o, m, nbytes), st);
+    if (nbytes % 16 == 0 && all_aligned(o, m))
+      return kTableTable[m - 1](coeff, k, d, o, nbytes / 16, st);
+  }
+  return wide_fn(k, m)(coeff, k, m, d, o, frame_of(o, m, nbytes), st);
 }
 
 }  // namespace
@@ -456,27 +888,15 @@ int ec_xor_encode(const uint8_t* const* d_data, int k, uint8_t* d_parity, uint64
   if (!d_parity) return EC_EINVAL;
   for (int j = 0; j < k; ++j)
     if (!d_data[j]) return EC_EINVAL;
-  uint8_t ones[EC_MAX_K];
-  for (int j = 0; j < k; ++j) ones[j] = 1;  // 1*x = x: XOR parity via the generic path
   uint8_t* const out[1] = {d_parity};
-  const int skew = ec::common_skew(out, 1, -1);
-  const bool same = ec::common_skew(d_data, k, skew) == skew;
-  uint64_t head = skew ? 16u - (uint64_t)skew : 0;
-  if (head > nbytes) head = nbytes;
-  int s = EC_OK;
-  if (head) s = ec::launch_generic(ones, k, 1, d_data, out, 0, head, st);
-  const uint64_t n16 = (nbytes - head) / 16;
-  if (s == EC_OK && n16) {
-    const uint8_t* da[EC_MAX_K];
-    for (int j = 0; j < k; ++j) da[j] = d_data[j] + head;
-    uint8_t* const oa[1] = {d_parity + head};
-    s = same && k <= ec::kFastMaxK ? ec::kXorTable[k - 1](da, d_parity + head, n16, st)
-                                   : ec::kWideTable[0](ones, k, da, oa, n16, st);
+  if (k > ec::kFastMaxK || nbytes < 16) {
+    uint8_t ones[EC_MAX_K];
+    for (int j = 0; j < k; ++j) ones[j] = 1;  // 1*x = x
+    return ec::matvec(ones, k, 1, d_data, out, nbytes, st);
   }
-  const uint64_t done = head + n16 * 16;
-  if (s == EC_OK && done < nbytes)
-    s = ec::launch_generic(ones, k, 1, d_data, out, done, nbytes - done, st);
-  return s;
+  if (nbytes % 16 == 0 && ec::all_aligned(d_data, k) && ec::all_aligned(out, 1))
+    return ec::kXorTable[k - 1](d_data, d_parity, nbytes / 16, st);
+  return ec::kAnyXorTable[k - 1](d_data, d_parity, ec::frame_of(out, 1, nbytes), st);
 }
 
 int ec_rs_encode(const uint8_t* coeff, int k, int m, const uint8_t* const* d_data,

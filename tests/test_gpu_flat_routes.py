@@ -1,0 +1,124 @@
+"""GPU parity of the flat calls' routes: sizes and alignments at the edges of
+the one-launch kernels for any shards, the matrix-core kernels for wide codes
+and the rules between them, each against the CPU encoder (pinned to the scalar
+oracle).  Integer work, so the bar is byte equality."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 0x5A
+
+
+def _carve(dev, arrays, offsets):
+    """Device views at the given offsets (mod 16) into one guarded arena each."""
+    views, arenas = [], []
+    for a, off in zip(arrays, offsets):
+        arena = torch.full((a.size + 64,), GUARD, dtype=torch.uint8, device=dev)
+        base = (off - arena.data_ptr()) % 16 + 16
+        view = arena[base: base + a.size]
+        view.copy_(torch.from_numpy(a))
+        views.append(view)
+        arenas.append((arena, base))
+    return views, arenas
+
+
+def _check(pkg, dev, k, m, n, in_off, out_off, coeff=None, data=None, seed=0):
+    rng = np.random.default_rng([k, m, n, seed])
+    host = data if data is not None else [rng.integers(0, 256, n, dtype=np.uint8) for _ in range(k)]
+    C = oracle.cauchy(k, m) if coeff is None else coeff
+    shards, _ = _carve(dev, host, [in_off(j) for j in range(k)])
+    outs, arenas = _carve(dev, [np.zeros(n, np.uint8)] * m, [out_off(i) for i in range(m)])
+    pkg.matvec(C, shards, out=outs)
+    torch.cuda.synchronize()
+    want = [np.empty(n, np.uint8) for _ in range(m)]
+    oracle.fast_rs_encode(C, host, want)
+    for i, ((arena, base), w) in enumerate(zip(arenas, want)):
+        got = arena.cpu().numpy()
+        assert np.array_equal(got[base: base + n], w), f"RS({k},{m}) n={n} output {i}"
+        assert (got[:base] == GUARD).all() and (got[base + n:] == GUARD).all(), \
+            f"RS({k},{m}) n={n} output {i}: bytes around it changed"
+
+
+# unrolled tables in registers / in LDS, any_kernel's five to eight outputs,
+# m <= 4 and k > 16, the deep codes with their bit matrix in registers / in LDS
+SHAPES = [(1, 1), (6, 3), (16, 4), (12, 8), (5, 5), (17, 1), (20, 4), (32, 3),
+          (13, 6), (24, 8), (31, 9), (32, 16), (4, 12)]
+
+
+@pytest.mark.parametrize("k,m", SHAPES)
+def test_sizes_at_chunk_and_step_edges(pkg, dev, k, m):
+    for n in [1, 15, 16, 17, 31, 32, 33, 511, 512, 513, 1024, 2047, 2049, 4096 + 5]:
+        _check(pkg, dev, k, m, n, lambda j: 0, lambda i: 0)
+
+
+@pytest.mark.parametrize("k,m", SHAPES)
+@pytest.mark.parametrize("n", [16, 29, 47, 1000, 4133])
+def test_every_shard_at_its_own_offset(pkg, dev, k, m, n):
+    _check(pkg, dev, k, m, n, lambda j: (5 * j + 3) % 16, lambda i: (7 * i + 1) % 16)
+    _check(pkg, dev, k, m, n, lambda j: 9, lambda i: 9)        # one offset for all
+    _check(pkg, dev, k, m, n, lambda j: 4 * j % 16, lambda i: 0)   # aligned outputs
+
+
+@pytest.mark.parametrize("k,m", [(6, 9), (17, 1), (10, 12), (20, 5), (10, 6), (6, 8), (20, 4),
+                                 (24, 8), (16, 16)])
+def test_both_sides_of_the_table_rule(pkg, dev, k, m):
+    """Shards of 2 MiB (matrix cores) and just above (where the tables pay:
+    RS(6,9) to RS(6,8))."""
+    for n in [2 << 20, (2 << 20) + 16, (2 << 20) + 33]:
+        _check(pkg, dev, k, m, n, lambda j: 0, lambda i: 0)
+    _check(pkg, dev, k, m, (2 << 20) + 16, lambda j: 4 * j % 16, lambda i: 0)
+
+
+@pytest.mark.parametrize("m", [1, 4, 7, 16])
+def test_sums_of_256_ones(pkg, dev, m):
+    """32 equal coefficients whose bit matrix has a row of ones: on shards of
+    0xFF that row's sum is 256, one more than two bytes per accumulator allow."""
+    def full_row(c):
+        products = [int(oracle.gf_mul(c, 1 << b)) for b in range(8)]
+        return any(all(p >> bit & 1 for p in products) for bit in range(8))
+    c = next(c for c in range(1, 256) if full_row(c))
+    coeff = np.full((m, 32), c, np.uint8)
+    coeff[m // 2:] = oracle.cauchy(32, m)[m // 2:]
+    n = 1500
+    ones = [np.full(n, 0xFF, np.uint8) for _ in range(32)]
+    ones[5][700:] = 3   # both kinds of column next to each other
+    for co in (coeff, np.full((m, 32), c, np.uint8)):
+        _check(pkg, dev, 32, m, n, lambda j: 0, lambda i: 0, coeff=co, data=ones)
+
+
+@pytest.mark.parametrize("k,m", [(6, 3), (10, 6), (24, 8), (20, 4)])
+@pytest.mark.parametrize("offset", [0, 5])
+def test_output_over_an_input(pkg, dev, k, m, offset):
+    """Outputs in place of the first inputs: each byte depends on its own column only."""
+    n = 40_007
+    rng = np.random.default_rng(k)
+    host = [rng.integers(0, 256, n, dtype=np.uint8) for _ in range(k)]
+    shards, _ = _carve(dev, host, [offset] * k)
+    e = min(k, m)
+    C = oracle.cauchy(k, e)
+    pkg.matvec(C, shards, out=shards[:e])
+    want = [np.empty(n, np.uint8) for _ in range(e)]
+    oracle.fast_rs_encode(C, host, want)
+    torch.cuda.synchronize()
+    for i in range(e):
+        assert np.array_equal(shards[i].cpu().numpy(), want[i])
+
+
+@pytest.mark.parametrize("k", [1, 2, 5, 16, 17, 32])
+def test_xor_any_shards(pkg, dev, k):
+    for n in [1, 16, 17, 1023, 1040, 70_001]:
+        for off in (lambda j: 0, lambda j: (3 * j + 1) % 16):
+            rng = np.random.default_rng([k, n])
+            host = [rng.integers(0, 256, n, dtype=np.uint8) for _ in range(k)]
+            shards, _ = _carve(dev, host, [off(j) for j in range(k)])
+            outs, arenas = _carve(dev, [np.zeros(n, np.uint8)], [off(2)])
+            pkg.xor_encode(shards, out=outs[0])
+            torch.cuda.synchronize()
+            got = arenas[0][0].cpu().numpy()
+            base = arenas[0][1]
+            assert np.array_equal(got[base: base + n], np.bitwise_xor.reduce(host))
+            assert (got[:base] == GUARD).all() and (got[base + n:] == GUARD).all()
