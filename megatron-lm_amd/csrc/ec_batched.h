@@ -18,7 +18,7 @@ namespace {
 // across the workgroup (scalar loads).
 //
 // The product launches one-wavefront workgroups with one 16-byte chunk per
-// lane, one 1 KiB tile of one stripe per workgroup (kBatchBlock, U = 1).
+// lane, one 1 KiB tile of one stripe per workgroup (kBatchBlock).
 // Measured on MI355X (HBM traffic, GB/s) against the former launcher
 // (256-lane workgroups walking 8-16 KiB of a stripe; four chunks per lane for
 // k <= 8 and units that are a multiple of 16 KiB): config 5's RS(12,4) over
@@ -41,7 +41,7 @@ struct BatchArgs {
                          // unit_bytes (0 = no copy); read only when the kernel copies
   PermTab tab[M][K];
   uint32_t unit_bytes;
-  uint32_t tiles_per_unit;   // tiles of B*U*16 bytes in a unit (B lanes)
+  uint32_t tiles_per_unit;   // tiles of B * 16 bytes in a unit (B lanes)
   uint32_t tiles_per_block;  // consecutive tiles one workgroup walks
   uint32_t blocks_per_unit;  // ceil(tiles_per_unit / tiles_per_block)
   FastDiv by_blocks;         // division by blocks_per_unit
@@ -50,16 +50,35 @@ struct BatchArgs {
   FastDiv by_groups;         // division by rest_groups
 };
 
-// Zeros in device memory, read-only: on the fast path a unit that ended
-// before the current tile is read from here instead of branching, so the
-// tile's k loads stay unconditional.  (Covers a tile of B * U * 16 bytes for
-// B * U <= 1024.)
-__device__ __align__(16) uint8_t g_zero_tile[1024 * 16] = {0};
+// When the tables go to LDS.  Behind the unit loads, so that the two latencies
+// overlap (RS(12,4) over ragged 64 KiB units 1328 -> 1319 us, RS(6,3) over
+// 1 MiB units 587 -> 581, RS(4,2) over 300 small tensors in 4 KiB units 4.4 ->
+// 3.9); but before them for the codes of eight and more units whose tables
+// then go on to registers (RS(8,2) over ragged 64 KiB units 346 -> 336).
+template <int K, int M, bool COPY>
+constexpr bool early_tables() {
+  return tables_in_registers<K, M>() && K >= 8 && !COPY;
+}
+
+// Two outputs of eight to ten units run fastest with three waves per SIMD:
+// RS(8,2) 336 us against 345 with the four that its registers allow, RS(10,2)
+// 333 against 375 with the two that it takes by itself.  Codes with more
+// outputs keep theirs (RS(12,4) with three 1392 against 1328, RS(6,3) 606 /
+// 587, RS(10,4) 403 / 383; five spill).
+template <int K, int M, bool COPY>
+constexpr bool three_waves() {
+  return early_tables<K, M, COPY>() && M == 2;
+}
+
+// Zeros in device memory, read-only: a unit that ended before the current tile
+// is read from here instead of branching, so the tile's k loads stay
+// unconditional.
+__device__ __align__(16) uint8_t g_zero_tile[1024] = {0};
 
 // Where tile_full's stores of outputs that ended before the tile point
 // (their stores are dropped by the range check of store_wave_if, so nothing
 // is written; a valid address all the same).
-__device__ __align__(16) uint8_t g_sink_tile[1024 * 16];
+__device__ __align__(16) uint8_t g_sink_tile[1024];
 
 // Store of 16 bytes at base + rel for tile_full (base wave-uniform); with
 // WAVE a store with keep false is dropped (store_wave_if).
@@ -102,8 +121,8 @@ __device__ __forceinline__ void tile_store(uint8_t* base, uint32_t rel, const ui
 // way: 3934 -> 4358 with WAVE, 4029 with global loads and sc1 buffer stores.
 template <int K, int M, int U, bool COPY, int B, bool WAVE>
 __device__ __forceinline__ void tile_full(const uint8_t* const (&src)[K], uint8_t* const (&dst)[M],
-                                          uint8_t* const (&cpy)[K],
-                                          const PermTab (&tab)[M][K], uint32_t keep = ~0u) {
+                                          uint8_t* const (&cpy)[K], const PermTab& mine,
+                                          PermTab (&tab)[M][K], uint32_t keep = ~0u) {
   static_assert(B * U * 16 <= sizeof(g_zero_tile), "tile larger than the zero tile");
   uint4 x[U][K];
 #pragma unroll
@@ -113,6 +132,7 @@ __device__ __forceinline__ void tile_full(const uint8_t* const (&src)[K], uint8_
     for (int j = 0; j < K; ++j)
       x[u][j] = WAVE ? load_wave(src[j], rel) : load_stream(src[j] + rel);
   }
+  if constexpr (WAVE && !early_tables<K, M, COPY>()) put_table<K, M>(tab, mine);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t rel = (u * B + threadIdx.x) * 16u;
@@ -126,93 +146,6 @@ __device__ __forceinline__ void tile_full(const uint8_t* const (&src)[K], uint8_
 #pragma unroll
       for (int j = 0; j < K; ++j)
         if (cpy[j]) tile_store<WAVE>(cpy[j], rel, x[u][j]);
-    }
-  }
-}
-
-// A full tile whose units are not all 16-byte aligned (tensors that are
-// views into a flat buffer at arbitrary offsets): one chunk per lane at a
-// time, each unit read through load_realign (one unaligned dwordx4 load for
-// a misaligned unit); the outputs are aligned.  A separate path from
-// tile_full on purpose: routing misaligned units through tile_full itself
-// (buffer loads at their byte addresses) changed the compiler's schedule of
-// the aligned path, config 5's encode 4145 -> 4250 us.
-template <int K, int M, int U, bool COPY, int B>
-__device__ __forceinline__ void tile_full_realign(const uint8_t* const (&src)[K],
-                                                  uint8_t* const (&dst)[M],
-                                                  uint8_t* const (&cpy)[K],
-                                                  const PermTab (&tab)[M][K]) {
-  constexpr int V = U >= 2 ? 2 : 1;  // chunks per lane in flight together
-#pragma unroll 1
-  for (int u0 = 0; u0 < U; u0 += V) {
-    uint4 x[V][K];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const uint32_t rel = ((u0 + v) * B + threadIdx.x) * 16u;
-#pragma unroll
-      for (int j = 0; j < K; ++j) x[v][j] = load_realign(src[j], rel);
-    }
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const uint32_t rel = ((u0 + v) * B + threadIdx.x) * 16u;
-      uint32_t acc[M][4] = {};
-      gf_matvec16<K, M>(acc, x[v], tab);
-#pragma unroll
-      for (int i = 0; i < M; ++i)
-        store_stream(dst[i] + rel, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
-      if constexpr (COPY) {
-#pragma unroll
-        for (int j = 0; j < K; ++j)
-          if (cpy[j]) store_stream(cpy[j] + rel, x[v][j]);
-      }
-    }
-  }
-}
-
-// Any other tile (a unit or output ending inside it, an absent unit, a
-// misaligned output): one unit at a time, descriptors re-read from memory,
-// byte-granular at the ends.  Kept as a rolled loop so that its registers
-// stay below the fast path's (the allocator takes the larger of the two).
-//
-// With COPY, each unit's chunk (zeros past its valid length) also goes to
-// its copy, over the whole unit_bytes.
-template <int K, int M, int U, bool COPY, int B>
-__device__ __forceinline__ void tile_edge(const BatchArgs<K, M>& a, uint32_t s, uint32_t base,
-                                          const PermTab (&tab)[M][K]) {
-  for (int u = 0; u < U; ++u) {
-    const uint32_t off = (base + u * B) * 16u;
-    if (off >= a.unit_bytes) continue;
-    uint32_t acc[M][4] = {};
-#pragma unroll 1
-    for (int j = 0; j < K; ++j) {
-      const uint8_t* dj = reinterpret_cast<const uint8_t*>(a.dptr[(uint64_t)s * K + j]);
-      uint32_t lj = dj ? a.dlen[(uint64_t)s * K + j] : 0u;
-      lj = lj < a.unit_bytes ? lj : a.unit_bytes;
-      uint4 xj = make_uint4(0u, 0u, 0u, 0u);
-      if (off < lj) {
-        xj = load_unit(dj, off, lj);
-        Fields f[4];
-#pragma unroll
-        for (int dd = 0; dd < 4; ++dd) f[dd] = fields(word(xj, dd));
-#pragma unroll
-        for (int i = 0; i < M; ++i) {
-          const PermTab t = tab[i][j];
-#pragma unroll
-          for (int dd = 0; dd < 4; ++dd) acc[i][dd] = mac1(acc[i][dd], t, f[dd]);
-        }
-      }
-      if constexpr (COPY) {
-        uint8_t* cj = reinterpret_cast<uint8_t*>(a.cptr[(uint64_t)s * K + j]);
-        if (cj) store_unit(cj, off, xj);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < M; ++i) {
-      uint8_t* pi = reinterpret_cast<uint8_t*>(a.pptr[(uint64_t)s * M + i]);
-      uint32_t li = a.olen ? a.olen[(uint64_t)s * M + i] : a.unit_bytes;
-      li = pi ? (li < a.unit_bytes ? li : a.unit_bytes) : 0u;
-      if (off < li)
-        store_unit_len(pi, off, li, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
     }
   }
 }
@@ -288,53 +221,120 @@ __device__ __forceinline__ void stripe_facts(Stripe<K, M, COPY>& st,
   }
 }
 
-// Tile t of stripe s through the path its contents need.  A tile is an edge
-// tile when some unit ends strictly inside it or some output does not cover
-// it (or an output is misaligned); a full tile with every unit aligned takes
-// tile_full, one with misaligned units tile_full_realign.
-template <int K, int M, int U, bool COPY, int B, bool WAVE>
+// Any other tile: units at any address, units or outputs that end inside it,
+// outputs at any address.  The K loads are in flight together all the same: a
+// unit that ends inside the tile is read at clamped addresses and its last
+// chunk shifted into place (clip_chunk), one that ended before it reads zeros.
+// A separate path from tile_full on purpose: routing misaligned units through
+// tile_full itself changed the compiler's schedule of the aligned path, config
+// 5's encode 4145 -> 4250 us.  Measured on MI355X against taking the units one
+// after the other, byte by byte at the ends and throughout where an output was
+// misaligned (us): RS(4,2) over 300 tensors of 256 B to 64 KiB in 4 KiB units
+// 7.0 -> 3.9; decode of 4 positions in place into 300 fp32 views of one flat
+// buffer, RS(12,4) in 64 KiB units 2208 -> 619 (1.46 -> 5.2 TB/s of HBM
+// traffic), RS(6,3) in 1 MiB units 2237 -> 660; copying encode of 300 small
+// views 11.6 -> 4.6.
+template <int K, int M, bool COPY, int B>
+__device__ __forceinline__ void tile_any(const BatchArgs<K, M>& a, uint32_t s, uint32_t t,
+                                         const Stripe<K, M, COPY>& st, const PermTab& mine,
+                                         PermTab (&tab)[M][K]) {
+  static_assert(B == 64, "one wavefront: no barrier around shorts");
+  __shared__ uint4 shorts[K];   // units of less than 16 bytes
+  const auto& len = st.len;
+  const uint32_t lo = t * (B * 16u), hi = lo + B * 16u;
+  // Opaque here, so that nothing of this path is computed ahead of the branch,
+  // on tile_full's path too.
+  uint32_t lane = threadIdx.x * 16u, chunk = 16u;
+  asm volatile("" : "+v"(lane), "+s"(chunk));
+  const uint32_t off = lo + lane;
+  uint4 x[K];
+  bool has_short = false;
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    const bool read = len[j] > lo && len[j] >= chunk;   // uniform
+    const uint32_t last = len[j] - chunk;
+    x[j] = load_any((read ? st.d[j] : g_zero_tile) + (!read ? lane : off < last ? off : last));
+    has_short |= len[j] > lo && len[j] < chunk;
+  }
+  if constexpr (!early_tables<K, M, COPY>()) put_table<K, M>(tab, mine);
+  if (has_short) {   // a rolled loop over the descriptors in memory: rare, so kept small
+#pragma unroll 1
+    for (int j = 0; j < K; ++j) {
+      const uint8_t* d = reinterpret_cast<const uint8_t*>(a.dptr[(uint64_t)s * K + j]);
+      const uint32_t l = d ? a.dlen[(uint64_t)s * K + j] : 0u;
+      if (l < 16u && lane == 0u) shorts[j] = load_short(d, l < a.unit_bytes ? l : a.unit_bytes);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    if (len[j] <= lo || len[j] >= hi) continue;   // uniform
+    if (len[j] >= chunk) x[j] = clip_chunk(x[j], off, len[j]);
+    else if (lane == 0u) x[j] = shorts[j];   // the other lanes hold zeros
+  }
+  uint32_t acc[M][4] = {};
+  gf_matvec16<K, M>(acc, x, tab);
+  pin_products(acc);
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const uint4 v = make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+    if (st.olen[i] >= hi)
+      store_any(st.p[i] + off, v);
+    else if (st.olen[i] > lo)
+      store_clip(st.p[i], off, st.olen[i], v);
+  }
+  if constexpr (COPY) {   // a copy spans the whole unit
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+      if (st.c[j] && off < a.unit_bytes) store_any(st.c[j] + off, x[j]);
+  }
+}
+
+// Tile t of a stripe through the path its contents need: tile_full when every
+// address is aligned and no unit or output ends strictly inside the tile (and,
+// without WAVE, every output covers it), else tile_any.
+template <int K, int M, bool COPY, int B, bool WAVE>
 __device__ __forceinline__ void code_tile(const BatchArgs<K, M>& a, uint32_t s, uint32_t t,
-                                          const Stripe<K, M, COPY>& st,
-                                          const PermTab (&tab)[M][K]) {
-  constexpr uint32_t kTileBytes = B * U * 16u;
-  const uint32_t base = t * (B * U) + threadIdx.x;
+                                          const Stripe<K, M, COPY>& st, const PermTab& mine,
+                                          PermTab (&tab)[M][K]) {
+  constexpr uint32_t kTileBytes = B * 16u;
   const uint32_t lo = t * kTileBytes, hi = lo + kTileBytes;
+  bool any = !st.in_aligned || !st.out_aligned;
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    any |= st.len[j] > lo && st.len[j] < hi;
+    if (COPY) any |= st.c[j] && a.unit_bytes < hi;  // a copy always spans the unit
+  }
+#pragma unroll
+  for (int i = 0; i < M; ++i)
+    any |= WAVE ? st.olen[i] > lo && st.olen[i] < hi : st.olen[i] < hi;
+  if (any) {
+    tile_any<K, M, COPY, B>(a, s, t, st, mine, tab);
+    return;
+  }
   const uint8_t* src[K];
   uint8_t* dst[M];
   uint8_t* cpy[K];
-  bool edge = !st.out_aligned;
 #pragma unroll
   for (int j = 0; j < K; ++j) {
     src[j] = st.len[j] >= hi ? st.d[j] + lo : g_zero_tile;
-    edge |= st.len[j] > lo && st.len[j] < hi;
     cpy[j] = st.c[j] ? st.c[j] + lo : nullptr;
-    if (COPY) edge |= st.c[j] && a.unit_bytes < hi;  // a copy always spans the unit
   }
   // With WAVE an output that ended at or before lo is dropped from the full
-  // path (keep); only an output ending strictly inside the tile makes it an
-  // edge tile.  The realigning path has no dropped stores: there any output
-  // short of hi makes an edge tile, as without WAVE.
+  // path (keep).
   uint32_t keep = 0;
-  bool short_out = false;
 #pragma unroll
   for (int i = 0; i < M; ++i) {
     const bool covers = st.olen[i] >= hi;
     dst[i] = covers ? st.p[i] + lo : g_sink_tile;
     keep |= (uint32_t)covers << i;
-    short_out |= !covers;
-    edge |= st.olen[i] > lo && st.olen[i] < hi;
   }
-  if (!WAVE || !st.in_aligned) edge |= short_out;
-  if (edge)
-    tile_edge<K, M, U, COPY, B>(a, s, base, tab);
-  else if (st.in_aligned)
-    tile_full<K, M, U, COPY, B, WAVE>(src, dst, cpy, tab, keep);
-  else
-    tile_full_realign<K, M, U, COPY, B>(src, dst, cpy, tab);
+  tile_full<K, M, 1, COPY, B, WAVE>(src, dst, cpy, mine, tab, keep);
 }
 
-template <int K, int M, int U, bool COPY, int B>
-__global__ void __launch_bounds__(B) batched_kernel(const BatchArgs<K, M> a) {
+template <int K, int M, bool COPY, int B>
+__global__ void __launch_bounds__(B)
+__attribute__((amdgpu_waves_per_eu(three_waves<K, M, COPY>() ? 3 : 1,
+                                   three_waves<K, M, COPY>() ? 3 : 8))) batched_kernel(const BatchArgs<K, M> a) {
   // The span this workgroup takes (uniform: a scalar branch); the grid is
   // rounded up to whole slices, and the few workgroups past the last span
   // return before any work.
@@ -347,11 +347,13 @@ __global__ void __launch_bounds__(B) batched_kernel(const BatchArgs<K, M> a) {
   const uint32_t t1 = min(t0 + a.tiles_per_block, a.tiles_per_unit);
   StripeDesc<K, M, COPY> r;
   read_stripe(r, a, s);
-  __shared__ PermTab tab[M][K];
-  stage_tables<K, M>(tab, a.tab);
+  __shared__ PermTab tab[M][K];   // filled by code_tile, behind its unit loads
+  PermTab mine;
+  if constexpr (early_tables<K, M, COPY>()) stage_tables<K, M>(tab, a.tab);
+  else mine = fetch_table<K, M>(a.tab);
   Stripe<K, M, COPY> st;
   stripe_facts(st, r, a.unit_bytes);
-  for (uint32_t t = t0; t < t1; ++t) code_tile<K, M, U, COPY, B, true>(a, s, t, st, tab);
+  for (uint32_t t = t0; t < t1; ++t) code_tile<K, M, COPY, B, true>(a, s, t, st, mine, tab);
 }
 
 // ---- large units: the full tiles and the rest, as two kernels ----------
@@ -473,12 +475,13 @@ __global__ void __launch_bounds__(B) batched_full_kernel(const BatchArgs<K, M> a
     }
 #pragma unroll
     for (int i = 0; i < M; ++i) dst[i] = st.p[i] + lo;
-    tile_full<K, M, 1, false, B, false>(src, dst, cpy, tab);
+    tile_full<K, M, 1, false, B, false>(src, dst, cpy, PermTab{}, tab);
   }
 }
 
 template <int K, int M, int B>
 __global__ void __launch_bounds__(B) batched_rest_kernel(const BatchArgs<K, M> a) {
+  static_assert(early_tables<K, M, false>(), "the tables are staged here, once");
   const uint32_t s = fast_div(blockIdx.x, a.by_groups);
   const uint32_t g = blockIdx.x - s * a.rest_groups;
   StripeDesc<K, M, false> r;
@@ -511,12 +514,12 @@ __global__ void __launch_bounds__(B) batched_rest_kernel(const BatchArgs<K, M> a
         }
       }
     }
-    code_tile<K, M, 1, false, B, false>(a, s, t, st, tab);
+    code_tile<K, M, false, B, false>(a, s, t, st, PermTab{}, tab);
   }
 }
 
-template <int K, int M, int U, bool COPY, int B>
-int launch_batched_u(const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
+template <int K, int M, bool COPY, int B>
+int launch_batched_b(const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
                      const uint64_t* pptr, const uint32_t* olen, const uint64_t* cptr,
                      uint32_t n_stripes, uint32_t unit_bytes, hipStream_t st) {
   BatchArgs<K, M> a;
@@ -529,7 +532,7 @@ int launch_batched_u(const uint8_t* coeff, const uint64_t* dptr, const uint32_t*
     for (int j = 0; j < K; ++j) a.tab[i][j] = perm_tab(coeff[i * K + j]);
   const uint32_t unit16 = unit_bytes / 16u;
   a.unit_bytes = unit_bytes;
-  a.tiles_per_unit = (unit16 + B * U - 1) / (B * U);
+  a.tiles_per_unit = (unit16 + B - 1) / B;
   // One tile per workgroup; spans of consecutive tiles only to keep the grid
   // below 2^30 workgroups.
   const uint64_t total_tiles = (uint64_t)n_stripes * a.tiles_per_unit;
@@ -539,12 +542,12 @@ int launch_batched_u(const uint8_t* coeff, const uint64_t* dptr, const uint32_t*
   a.tiles_per_block = (uint32_t)tpb;
   a.blocks_per_unit = (a.tiles_per_unit + a.tiles_per_block - 1) / a.tiles_per_block;
   a.by_blocks = make_fastdiv(a.blocks_per_unit);
-  const bool split = !COPY && U == 1 && split_pays<K, M>() && a.tiles_per_block == 1 &&
+  const bool split = !COPY && split_pays<K, M>() && a.tiles_per_block == 1 &&
                      unit_bytes >= kSplitMinUnit && unit_bytes < kSplitMaxUnit;
   const uint64_t blocks = span_grid(a.grid, (uint64_t)n_stripes * a.blocks_per_unit,
                                     split ? 0u : slice_shift_for(unit_bytes, COPY));
   if (blocks == 0) return EC_ERANGE;
-  if constexpr (!COPY && U == 1 && split_pays<K, M>()) {
+  if constexpr (!COPY && split_pays<K, M>()) {
     if (split) {
       // Enough rest workgroups to fill the chip when whole stripes are
       // misaligned (about 8192 in all), at most one per tile.
@@ -561,7 +564,7 @@ int launch_batched_u(const uint8_t* coeff, const uint64_t* dptr, const uint32_t*
       return hip_status();
     }
   }
-  hipLaunchKernelGGL((batched_kernel<K, M, U, COPY, B>), dim3((unsigned)blocks), dim3(B), 0,
+  hipLaunchKernelGGL((batched_kernel<K, M, COPY, B>), dim3((unsigned)blocks), dim3(B), 0,
                      st, a);
   return hip_status();
 }

@@ -21,7 +21,7 @@ template <int K, int M>
 int launch_batched(const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
                    const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,
                    uint32_t unit_bytes, hipStream_t st) {
-  return launch_batched_u<K, M, 1, false, kBatchBlock>(coeff, dptr, dlen, pptr, olen, nullptr,
+  return launch_batched_b<K, M, false, kBatchBlock>(coeff, dptr, dlen, pptr, olen, nullptr,
                                                        n_stripes, unit_bytes, st);
 }
 

@@ -16,7 +16,7 @@ template <int K, int M>
 int launch_batched_copy(const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
                         const uint64_t* pptr, const uint64_t* cptr, uint32_t n_stripes,
                         uint32_t unit_bytes, hipStream_t st) {
-  return launch_batched_u<K, M, 1, true, kBatchBlock>(coeff, dptr, dlen, pptr, nullptr, cptr,
+  return launch_batched_b<K, M, true, kBatchBlock>(coeff, dptr, dlen, pptr, nullptr, cptr,
                                                       n_stripes, unit_bytes, st);
 }
 

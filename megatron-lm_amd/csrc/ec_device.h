@@ -132,8 +132,15 @@ __device__ __forceinline__ void store_stream(void* p, const uint4& v) {
   __builtin_nontemporal_store(w, (global_u32x4*)(uintptr_t)p);
 }
 
-// The same at any byte address (a vector type of alignment 1: gfx950 takes
-// the single dwordx4 access, see load_realign).
+// The same at any byte address: the vector type has alignment 1, so the
+// compiler does not assume an alignment; for gfx950 it emits the single dwordx4
+// all the same, as it does for any 16-byte memcpy from a byte pointer, since
+// the ROCm driver runs compute queues with unaligned memory access enabled.
+// Exactly the 16 bytes asked for are touched.  Measured on MI355X against
+// loading the two aligned blocks around the bytes and shifting them into place
+// (HBM traffic, TB/s, 600 fp32 views of one flat buffer through the batched
+// kernels): RS(12,4) in 64 KiB units 4.66 -> 5.88, RS(6,3) in 1 MiB units 4.88
+// -> 5.94 (6.15-6.65 for aligned copies of the same tensors).
 typedef uint32_t u32x4_unaligned __attribute__((ext_vector_type(4), aligned(1)));
 typedef __attribute__((address_space(1))) u32x4_unaligned global_u32x4_unaligned;
 
@@ -196,7 +203,21 @@ __device__ __forceinline__ void store_wave_if(void* base, uint32_t lane_off, con
 // Copy the m x k permute tables from the kernel arguments into LDS, where
 // the unrolled loops read them as wave-uniform broadcasts straight into
 // VGPRs (v_perm_b32 may read only one SGPR, so tables held in SGPRs cost a
-// v_mov per use and spill beyond ~100 SGPRs).
+// v_mov per use and spill beyond ~100 SGPRs).  In two parts, so that a kernel
+// can issue its shard loads between them and wait for both together.
+template <int K, int M>
+__device__ __forceinline__ PermTab fetch_table(const PermTab (&src)[M][K]) {
+  const uint32_t t = threadIdx.x < M * K ? threadIdx.x : M * K - 1;
+  return src[t / K][t % K];
+}
+
+template <int K, int M>
+__device__ __forceinline__ void put_table(PermTab (&dst)[M][K], const PermTab& mine) {
+  const uint32_t t = threadIdx.x;
+  if (t < M * K) dst[t / K][t % K] = mine;
+  __syncthreads();
+}
+
 template <int K, int M>
 __device__ __forceinline__ void stage_tables(PermTab (&dst)[M][K], const PermTab (&src)[M][K]) {
   const int t = threadIdx.x;
@@ -328,63 +349,105 @@ constexpr int kWidePair() {
 }
 
 // 16 bytes at base + off, where off is a multiple of 16 and base may have any
-// alignment r = base mod 16 (uniform: it depends on the shard only).  r = 0
-// is the aligned dwordx4 load; otherwise one dwordx4 load at the unaligned
-// address (the vector type below has alignment 1, so the compiler does not
-// assume an alignment; for gfx950 it emits the single dwordx4 all the same,
-// as it does for any 16-byte memcpy from a byte pointer, since the ROCm
-// driver runs compute queues with unaligned memory access enabled),
-// non-temporal like the aligned one.  It reads exactly the 16
-// bytes asked for.  Measured on MI355X against the former form (the two
-// aligned blocks holding the bytes, shifted into place with
-// v_alignbyte_b32), HBM traffic, TB/s, one box: 600 fp32 tensor views of one
-// flat buffer (6.82 GB, 450 of them misaligned) through the batched kernels,
-// RS(12,4) in 64 KiB units 4.66 -> 5.88, RS(8,2) in 4 MiB units 3.51 ->
-// 4.15, RS(6,3) in 1 MiB units 4.88 -> 5.94 (6.15-6.65 for aligned copies of
-// the same tensors); RS(6,3) over six 64 MiB shards at skews 1-6 through the
-// wide kernel 5.24 -> 5.62.  Aligned inputs do not take this path.
+// alignment (uniform: it depends on the shard only), for the table kernel:
+// the aligned dwordx4 load, or one at the unaligned address.
 __device__ __forceinline__ uint4 load_realign(const uint8_t* base, uint64_t off) {
   if ((reinterpret_cast<uintptr_t>(base) & 15u) == 0) return load_stream(base + off);
   return load_any(base + off);
 }
 
 // ---------------------------------------------------------- unit access --
-// 16 bytes of a unit at byte offset off, zero beyond len.  A 16-byte-aligned
-// unit takes one dwordx4 load; the chunk that straddles len, and every chunk
-// of a misaligned unit, is read byte by byte, so nothing past len is read.
-__device__ __forceinline__ uint4 load_unit(const uint8_t* p, uint32_t off, uint32_t len) {
-  if (off + 16u <= len && (reinterpret_cast<uintptr_t>(p) & 15u) == 0)
-    return load_stream(p + off);
-  const global_u8* g = gptr(p);
-  uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int b = 0; b < 16; ++b)
-    if (off + b < len) w[b >> 2] |= (uint32_t)g[off + b] << (8 * (b & 3));
-  return make_uint4(w[0], w[1], w[2], w[3]);
+// 16 bytes of a unit of len bytes at byte offset off (a multiple of 16), at any
+// address, zeros past len, nothing past len read: the chunk that straddles len
+// is the unit's last 16 bytes shifted down.  In two parts, so that the loads
+// of several units are in flight together: load_any(clip_address(...)), then
+// clip_chunk on what came back; units of less than 16 bytes read zeros there
+// and come from load_short.
+__device__ __align__(16) const uint8_t g_zeros[16] = {0};
+
+__device__ __forceinline__ const uint8_t* clip_address(const uint8_t* p, uint32_t off,
+                                                       uint32_t len) {
+  if (len < 16u) return g_zeros;
+  return p + (off < len - 16u ? off : len - 16u);
 }
 
-// Store 16 parity bytes at byte offset off (byte stores if p is misaligned).
-__device__ __forceinline__ void store_unit(uint8_t* p, uint32_t off, const uint4& v) {
-  if ((reinterpret_cast<uintptr_t>(p) & 15u) == 0) {
-    store_stream(p + off, v);
-    return;
-  }
-  global_u8* g = gptr(p);
-#pragma unroll
-  for (int b = 0; b < 16; ++b) g[off + b] = (uint8_t)(word(v, b >> 2) >> (8 * (b & 3)));
+// v shifted down by n bytes (0 to 16 and more), zeros from above.
+__device__ __forceinline__ uint4 shift_down(uint4 v, uint32_t n) {
+  if (n & 8u) v = make_uint4(v.z, v.w, 0u, 0u);
+  if (n & 4u) v = make_uint4(v.y, v.z, v.w, 0u);
+  v = make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, n), __builtin_amdgcn_alignbyte(v.z, v.y, n),
+                 __builtin_amdgcn_alignbyte(v.w, v.z, n), __builtin_amdgcn_alignbyte(0u, v.w, n));
+  return n < 16u ? v : make_uint4(0u, 0u, 0u, 0u);
 }
 
-// Store the bytes of v that fall below len at byte offset off of p.
-__device__ __forceinline__ void store_unit_len(uint8_t* p, uint32_t off, uint32_t len,
-                                               const uint4& v) {
-  if (off + 16u <= len) {
-    store_unit(p, off, v);
-    return;
+// The first 16 bytes of a unit of len < 16 bytes, from two loads of 8, 4 or 2
+// bytes that overlap in the middle.
+template <typename T>
+__device__ inline uint64_t load_pair(const uint8_t* p, uint32_t len) {
+  typedef T __attribute__((aligned(1))) any_t;
+  typedef __attribute__((address_space(1))) any_t global_any;
+  constexpr uint32_t kW = sizeof(T);
+  const uint64_t lo = *(const global_any*)(uintptr_t)p;
+  const uint64_t hi = *(const global_any*)(uintptr_t)(p + (len - kW));
+  return lo | (hi << (8u * (len - kW)));   // kW < 8: the overlap holds equal bytes
+}
+
+__device__ __forceinline__ uint4 load_short(const uint8_t* p, uint32_t len) {
+  uint64_t lo = 0, hi = 0;
+  if (len >= 8u) {
+    typedef uint64_t __attribute__((aligned(1))) any64;
+    typedef __attribute__((address_space(1))) any64 global_any64;
+    lo = *(const global_any64*)(uintptr_t)p;
+    const uint64_t last = *(const global_any64*)(uintptr_t)(p + (len - 8u));
+    hi = len == 8u ? 0u : last >> (8u * (16u - len));
+  } else if (len >= 4u) {
+    lo = load_pair<uint32_t>(p, len);
+  } else if (len >= 2u) {
+    lo = load_pair<uint16_t>(p, len);
+  } else if (len == 1u) {
+    lo = gptr(p)[0];
   }
-  global_u8* g = gptr(p);
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+}
+
+__device__ __forceinline__ uint4 clip_chunk(const uint4& v, uint32_t off, uint32_t len) {
+  return off + 16u <= len ? v : shift_down(v, off + 16u - len);
+}
+
+// Both parts at once, any unit.
+__device__ __forceinline__ uint4 load_clip(const uint8_t* p, uint32_t off, uint32_t len) {
+  const uint4 v = load_any(clip_address(p, off, len));
+  if (len < 16u) return off < len ? load_short(p, len) : v;
+  return clip_chunk(v, off, len);
+}
+
+// Bytes [from, to) of v at p, one at a time.
+__device__ __forceinline__ void store_bytes(uint8_t* p, uint32_t from, uint32_t to, uint4 v) {
+#pragma unroll 1
+  for (uint32_t b = 0; b < to; ++b) {   // shifted down, so that no register is indexed
+    if (b >= from) gptr(p)[b] = (uint8_t)v.x;
+    v = make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, 1), __builtin_amdgcn_alignbyte(v.z, v.y, 1),
+                   __builtin_amdgcn_alignbyte(v.w, v.z, 1), v.w >> 8);
+  }
+}
+
+// The bytes of v that fall below len at byte offset off of p.
+__device__ __forceinline__ void store_clip(uint8_t* p, uint32_t off, uint32_t len,
+                                           const uint4& v) {
+  if (off + 16u <= len)
+    store_any(p + off, v);
+  else if (off < len)
+    store_bytes(p + off, 0u, len - off, v);
+}
+
+// All products here, not each output's sunk into the branches of its store
+// (RS(12,4) in any_kernel: the tables would stay live in 340 registers).
+template <int M>
+__device__ __forceinline__ void pin_products(uint32_t (&acc)[M][4]) {
 #pragma unroll
-  for (int b = 0; b < 16; ++b)
-    if (off + b < len) g[off + b] = (uint8_t)(word(v, b >> 2) >> (8 * (b & 3)));
+  for (int i = 0; i < M; ++i)
+#pragma unroll
+    for (int dd = 0; dd < 4; ++dd) asm volatile("" : "+v"(acc[i][dd]));
 }
 
 // ---------------------------------------------------------- host launch --

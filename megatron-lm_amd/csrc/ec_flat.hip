@@ -227,14 +227,8 @@ __device__ __forceinline__ Step step_of(const Frame& f, uint64_t step, uint32_t 
 
 __device__ __forceinline__ bool whole(const Step& s) { return s.to - s.from == 16u; }
 
-// Bytes [from, to) of v, one at a time.
-__device__ __forceinline__ void store_edge(uint8_t* p, const Step& s, uint4 v) {
-#pragma unroll 1
-  for (uint32_t b = 0; b < s.to; ++b) {   // shifted down, so that no register is indexed
-    if (b >= s.from) gptr(p)[b] = (uint8_t)v.x;
-    v = make_uint4(__builtin_amdgcn_alignbyte(v.y, v.x, 1), __builtin_amdgcn_alignbyte(v.z, v.y, 1),
-                   __builtin_amdgcn_alignbyte(v.w, v.z, 1), v.w >> 8);
-  }
+__device__ __forceinline__ void store_edge(uint8_t* p, const Step& s, const uint4& v) {
+  store_bytes(p, s.from, s.to, v);
 }
 
 template <int M>
@@ -249,16 +243,6 @@ __device__ __forceinline__ void store_outputs(uint8_t* const (&out)[M], uint64_t
     for (int i = 0; i < M; ++i)
       store_edge(out[i] + off, s, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
   }
-}
-
-// All products here, not each output's sunk into the branches of its store
-// (RS(12,4) in any_kernel: the tables would stay live in 340 registers).
-template <int M>
-__device__ __forceinline__ void pin_products(uint32_t (&acc)[M][4]) {
-#pragma unroll
-  for (int i = 0; i < M; ++i)
-#pragma unroll
-    for (int dd = 0; dd < 4; ++dd) asm volatile("" : "+v"(acc[i][dd]));
 }
 
 template <int K, int M>
@@ -813,10 +797,7 @@ inline Frame frame_of(uint8_t* const* o, int m, uint64_t nbytes) {
 }
 
 // Whether the permute tables take fewer cycles than the matrix cores for a
-// code past the unrolled kernels: SIMD cycles per 512 byte columns, 4 per VALU
-// op (1.125 k m + 1.25 k ops per column against the transposes, expansions and
-// bit selects of ec_mfma.h) and 32 per MFMA; the two kinds measured as good as
-// additive.  Both kernels over 64 MiB shards (HBM traffic, TB/s, tables /
+// code past the unrolled kernels.  Both kernels over 64 MiB shards (HBM traffic, TB/s, tables /
 // matrix cores; * any_kernel's tables): RS(17,1) 6.03 / 5.48, RS(6,9) 5.59 /
 // 4.91, RS(4,16) 5.43 / 4.75, RS(10,10) 4.73 / 4.07, RS(20,5) 5.14 / 4.82,
 // RS(10,6) 5.95* / 4.82, RS(5,5) 5.92* / 5.02, RS(12,8) 5.17* / 5.24, and past

@@ -152,32 +152,62 @@ __global__ void __launch_bounds__(B) update_kernel(const UpdateArgs<K, M> a) {
     // is misaligned; parity bytes past the longest changed unit stay as they are
 #pragma unroll 1
     for (int u = 0; u < U; ++u) {
-      const uint32_t off = lo + (u * B + threadIdx.x) * 16u;
+      uint32_t off = lo + (u * B + threadIdx.x) * 16u;
+      asm volatile("" : "+v"(off));   // nothing of this path ahead of the branch
       if (off >= longest) continue;
+      uint4 pv[M];
+#pragma unroll
+      for (int i = 0; i < M; ++i) pv[i] = load_any(p[i] + off);
       uint32_t acc[M][4] = {};
+      // A loop over the descriptors in memory, four units' loads in flight at a
+      // time: few tiles, so kept small and below the vector path's registers.
+      constexpr int G = K < 4 ? K : 4;
+#pragma unroll 1
+      for (int j0 = 0; j0 < K; j0 += G) {
+        const uint8_t* n[G];
+        const uint8_t* o[G];
+        uint32_t l[G];
+        uint4 vn[G], vo[G];
 #pragma unroll
-      for (int j = 0; j < K; ++j) {
-        if (nw[j] == nullptr || off >= len[j]) continue;
-        const uint4 vn = load_unit(nw[j], off, len[j]);
-        const uint4 vo = load_unit(od[j], off, len[j]);
-        const uint4 dl = make_uint4(vn.x ^ vo.x, vn.y ^ vo.y, vn.z ^ vo.z, vn.w ^ vo.w);
-        Fields f[4];
+        for (int g = 0; g < G; ++g) {
+          const int j = j0 + g < K ? j0 + g : K - 1;
+          n[g] = reinterpret_cast<const uint8_t*>(a.nptr[(uint64_t)s * K + j]);
+          o[g] = reinterpret_cast<const uint8_t*>(a.optr[(uint64_t)s * K + j]);
+          const uint32_t lj = a.len[(uint64_t)s * K + j];
+          l[g] = n[g] && j0 + g < K ? (lj < a.unit_bytes ? lj : a.unit_bytes) : 0u;
+        }
 #pragma unroll
-        for (int dd = 0; dd < 4; ++dd) f[dd] = fields(word(dl, dd));
+        for (int g = 0; g < G; ++g) {
+          vn[g] = load_any(off < l[g] ? clip_address(n[g], off, l[g]) : g_zeros);
+          vo[g] = load_any(off < l[g] ? clip_address(o[g], off, l[g]) : g_zeros);
+        }
 #pragma unroll
-        for (int i = 0; i < M; ++i) {
-          asm volatile("" ::: "memory");
-          const PermTab tj = tab[i][j];
+        for (int g = 0; g < G; ++g) {
+          if (off >= l[g]) continue;
+          if (l[g] < 16u) {
+            vn[g] = load_short(n[g], l[g]);
+            vo[g] = load_short(o[g], l[g]);
+          } else {
+            vn[g] = clip_chunk(vn[g], off, l[g]);
+            vo[g] = clip_chunk(vo[g], off, l[g]);
+          }
+          const uint4 dl = make_uint4(vn[g].x ^ vo[g].x, vn[g].y ^ vo[g].y, vn[g].z ^ vo[g].z,
+                                      vn[g].w ^ vo[g].w);
+          Fields f[4];
 #pragma unroll
-          for (int dd = 0; dd < 4; ++dd) acc[i][dd] = mac1(acc[i][dd], tj, f[dd]);
+          for (int dd = 0; dd < 4; ++dd) f[dd] = fields(word(dl, dd));
+#pragma unroll
+          for (int i = 0; i < M; ++i) {
+            const PermTab tj = tab[i][j0 + g];
+#pragma unroll
+            for (int dd = 0; dd < 4; ++dd) acc[i][dd] = mac1(acc[i][dd], tj, f[dd]);
+          }
         }
       }
 #pragma unroll
-      for (int i = 0; i < M; ++i) {
-        const uint4 v = load_unit(p[i], off, a.unit_bytes);
-        store_unit(p[i], off, make_uint4(v.x ^ acc[i][0], v.y ^ acc[i][1], v.z ^ acc[i][2],
-                                         v.w ^ acc[i][3]));
-      }
+      for (int i = 0; i < M; ++i)
+        store_any(p[i] + off, make_uint4(pv[i].x ^ acc[i][0], pv[i].y ^ acc[i][1],
+                                         pv[i].z ^ acc[i][2], pv[i].w ^ acc[i][3]));
     }
   }
 }

@@ -141,13 +141,12 @@ __global__ void __launch_bounds__(B) batched_wide_kernel(const BatchWideArgs a) 
 #pragma unroll 1
       for (int j = 0; j < k; ++j) {
         if (off >= w.len[j]) continue;
-        wide_mac<M>(acc, load_unit(w.d[j], off, w.len[j]), &w.tab[j], k);
+        wide_mac<M>(acc, load_clip(w.d[j], off, w.len[j]), &w.tab[j], k);
       }
 #pragma unroll
       for (int i = 0; i < M; ++i)
-        if (off < w.plen[i])
-          store_unit_len(w.p[i], off, w.plen[i],
-                         make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
+        store_clip(w.p[i], off, w.plen[i],
+                   make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
     }
   }
 }
@@ -170,18 +169,18 @@ __global__ void __launch_bounds__(B) update_wide_kernel(const BatchWideArgs a) {
     uint32_t acc[M][4] = {};
     uint4 pv[M];  // the parity does not depend on the delta: load it first
 #pragma unroll
-    for (int i = 0; i < M; ++i) pv[i] = load_unit(w.p[i], off, a.unit_bytes);
+    for (int i = 0; i < M; ++i) pv[i] = load_any(w.p[i] + off);
 #pragma unroll 1
     for (int j = 0; j < k; ++j) {
       if (w.d[j] == nullptr || off >= w.len[j]) continue;  // unchanged unit, or past its end
-      const uint4 vn = load_unit(w.d[j], off, w.len[j]);
-      const uint4 vo = load_unit(w.o[j], off, w.len[j]);
+      const uint4 vn = load_clip(w.d[j], off, w.len[j]);
+      const uint4 vo = load_clip(w.o[j], off, w.len[j]);
       wide_mac<M>(acc, make_uint4(vn.x ^ vo.x, vn.y ^ vo.y, vn.z ^ vo.z, vn.w ^ vo.w),
                   &w.tab[j], k);
     }
 #pragma unroll
     for (int i = 0; i < M; ++i)
-      store_unit(w.p[i], off, make_uint4(pv[i].x ^ acc[i][0], pv[i].y ^ acc[i][1],
+      store_any(w.p[i] + off, make_uint4(pv[i].x ^ acc[i][0], pv[i].y ^ acc[i][1],
                                          pv[i].z ^ acc[i][2], pv[i].w ^ acc[i][3]));
   }
 }

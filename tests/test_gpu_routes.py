@@ -1,7 +1,7 @@
-"""GPU parity of the flat calls' routes: sizes and alignments at the edges of
-the one-launch kernels for any shards, the matrix-core kernels for wide codes
-and the rules between them, each against the CPU encoder (pinned to the scalar
-oracle).  Integer work, so the bar is byte equality."""
+"""GPU parity of the routes: sizes and alignments at the edges of the one-launch
+flat kernels, the matrix-core kernels for wide codes, the rules between them
+and the batched kernels' edge tiles, each against the CPU encoder or the scalar
+oracle.  Integer work, so the bar is byte equality."""
 import numpy as np
 import pytest
 import torch
@@ -122,3 +122,82 @@ def test_xor_any_shards(pkg, dev, k):
             base = arenas[0][1]
             assert np.array_equal(got[base: base + n], np.bitwise_xor.reduce(host))
             assert (got[:base] == GUARD).all() and (got[base + n:] == GUARD).all()
+
+
+# ------------------------------------------------------- batched edge tiles --
+
+@pytest.mark.parametrize("k,m,unit", [(4, 2, 1024), (12, 4, 1040), (8, 2, 4096), (6, 3, 16),
+                                      (16, 1, 2048), (20, 6, 1024)])
+@pytest.mark.parametrize("skew", [0, 1, 6])
+def test_units_of_every_length_around_the_chunk(pkg, dev, k, m, unit, skew):
+    """Tensors of 1 to 33 bytes and of lengths around a tile, aligned and back
+    to back at any byte, through encode, copying encode, decode in place and
+    update; bytes between the tensors stay."""
+    rng = np.random.default_rng([k, m, unit, skew])
+    sizes = list(range(1, 34)) + [unit - 1, unit, unit + 1, unit + 15, 2 * unit + 17, 1007, 1009,
+                                  1023, 1025, 1041]
+    rng.shuffle(sizes)
+    gap = 3 if skew else 0
+    starts, at = [], skew
+    for sz in sizes:
+        starts.append(at)
+        at += sz + gap if skew else -(-sz // 16) * 16
+    arena = torch.full((at + 64,), GUARD, dtype=torch.uint8, device=dev)
+    host = [rng.integers(0, 256, sz, dtype=np.uint8) for sz in sizes]
+    tensors = [arena[a: a + sz] for a, sz in zip(starts, sizes)]
+    for t, h in zip(tensors, host):
+        t.copy_(torch.from_numpy(h))
+    lay = pkg.StripeLayout(tensors, k, m, unit)
+
+    def expected(hs):
+        grid = []
+        for s in range(lay.n_stripes):
+            row = []
+            for j in range(k):
+                u = s * k + j
+                t, i = (int(lay.unit_tensor[u]), int(lay.unit_index[u])) if u < lay.n_units \
+                    else (-1, 0)
+                row.append(hs[t][i * unit: (i + 1) * unit] if t >= 0 else None)
+            grid.append(row)
+        return oracle.encode_batched(lay.coeff, grid, lay.host_len, unit)
+
+    parity = lay.encode()
+    torch.cuda.synchronize()
+    want = expected(host)
+    assert np.array_equal(parity.cpu().numpy(), want)
+
+    from megatron_lm_amd.checkpoint import GpuSliceCodec
+    _, slices = GpuSliceCodec(k, m, unit).encode(tensors)
+    for i in range(m):
+        assert np.array_equal(slices[k + i], want[:, i].reshape(-1))
+    for j in range(k):
+        units = np.zeros((lay.n_stripes, unit), np.uint8)
+        for s in range(lay.n_stripes):
+            u = s * k + j
+            if u < lay.n_units:
+                piece = host[int(lay.unit_tensor[u])][int(lay.unit_index[u]) * unit:][:unit]
+                units[s, : piece.size] = piece
+        assert np.array_equal(slices[j], units.reshape(-1))
+
+    before = arena.clone()
+    lost = sorted(int(x) for x in rng.choice(k + m, m, replace=False))
+    for p in lost:
+        if p < k:
+            for s in range(lay.n_stripes):
+                if s * k + p < lay.n_units:
+                    lay.unit_view(s * k + p).fill_(0xEE)
+        else:
+            parity[:, p - k].fill_(0xEE)
+    lay.decode(parity, lost)
+    torch.cuda.synchronize()
+    assert torch.equal(arena, before), f"lost {lost}"
+    assert np.array_equal(parity.cpu().numpy(), want)
+
+    changed = sorted(int(x) for x in rng.choice(lay.n_units, lay.n_units // 2, replace=False))
+    old = [lay.unit_view(u).clone() for u in changed]
+    for u in changed:
+        lay.unit_view(u).bitwise_xor_(0x6B)
+    lay.update(parity, changed, old)
+    torch.cuda.synchronize()
+    now = [t.cpu().numpy() for t in tensors]
+    assert np.array_equal(parity.cpu().numpy(), expected(now))
