@@ -803,12 +803,7 @@ inline Frame frame_of(uint8_t* const* o, int m, uint64_t nbytes) {
 // RS(10,6) 5.95* / 4.82, RS(5,5) 5.92* / 5.02, RS(12,8) 5.17* / 5.24, and past
 // the line RS(8,12) 4.92 / 5.40, RS(16,6) 4.87 / 5.55, RS(20,4) 5.60 / 6.04,
 // RS(16,8) 4.36 / 5.55, RS(24,8) 4.09 / 5.38, RS(32,16) 2.69 / 3.93.
-bool table_pays(int k, int m) {
-  const int kt = (k + kMfmaShards - 1) / kMfmaShards, mt = (m + kMfmaOutputs - 1) / kMfmaOutputs;
-  const int tables = 36 * k * m + 40 * k;
-  const int cores = 512 * kt * mt + 448 * kt + 240 * ((m + 1) / 2);
-  return tables <= cores;
-}
+bool table_pays(int k, int m) { return table_cost(k, m) <= core_cost(k, m); }
 
 // Up to this shard size too few waves run to be bound by either's arithmetic
 // and the matrix cores' shorter chains win for every code (2 MiB shards, us,

@@ -10,6 +10,7 @@
 #include <utility>
 
 #include "ec_device.h"
+#include "ec_mfma.h"
 #include "ec_update.h"
 
 namespace ec {
@@ -185,6 +186,152 @@ __global__ void __launch_bounds__(B) update_wide_kernel(const BatchWideArgs a) {
   }
 }
 
+// The encode and decode of wide codes on the matrix cores (ec_mfma.h): a wave
+// codes 512 bytes of every unit of a stripe per step, lane l and lane l + 32
+// the same columns of the even and the odd units.  A workgroup stages its
+// stripe's descriptors in LDS once for the steps it walks.  Units and outputs
+// at any address and of any length take the same path: a unit is read at
+// clamped addresses and the chunk that holds its end shifted into place.
+struct BatchCoreArgs {
+  const uint64_t* dptr;  // [n_stripes][k]
+  const uint32_t* dlen;  // [n_stripes][k]
+  const uint64_t* pptr;  // [n_stripes][m]
+  const uint32_t* olen;  // [n_stripes][m] valid output bytes, or null = whole units
+  MfmaCoeff coeff;
+  uint32_t unit_bytes;
+  uint32_t steps_per_unit;   // ceil(unit_bytes / 512)
+  uint32_t steps_per_block;  // consecutive steps one workgroup walks
+  uint32_t blocks_per_unit;
+  FastDiv by_blocks;         // division by blocks_per_unit
+  int k, m;
+};
+
+constexpr uint32_t kCoreStep = 512;   // bytes of each unit per wave and step
+
+template <int KH, int MH>
+struct CoreLds {
+  const uint8_t* d[EC_MAX_K];
+  uint32_t len[EC_MAX_K];
+  uint8_t* p[EC_MAX_M];
+  uint32_t plen[EC_MAX_M];
+  typename MfmaCode<KH, MH>::Lds code;
+};
+
+template <int KH, int MH, bool PAIR>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2)))
+batched_core_kernel(const BatchCoreArgs a) {
+  constexpr int KT = mfma_groups(KH), MT = mfma_tiles(MH);
+  constexpr uint32_t kWaves = kBlock / 64;
+  __shared__ CoreLds<KH, MH> w;
+  const uint32_t s = fast_div(blockIdx.x, a.by_blocks);
+  const uint32_t s0 = (blockIdx.x - s * a.blocks_per_unit) * a.steps_per_block;
+  const uint32_t s1 = min(s0 + a.steps_per_block, a.steps_per_unit);
+  const uint32_t t = threadIdx.x;
+  if (t < EC_MAX_K) {
+    const bool in = (int)t < a.k;
+    const uint64_t d = in ? a.dptr[(uint64_t)s * a.k + t] : 0u;
+    const uint32_t l = in ? a.dlen[(uint64_t)s * a.k + t] : 0u;
+    w.d[t] = reinterpret_cast<const uint8_t*>(d);
+    w.len[t] = d ? (l < a.unit_bytes ? l : a.unit_bytes) : 0u;
+  } else if (t >= 64 && t < 64 + EC_MAX_M) {
+    const uint32_t i = t - 64;
+    const bool in = (int)i < a.m;
+    const uint64_t q = in ? a.pptr[(uint64_t)s * a.m + i] : 0u;
+    const uint32_t l = !in ? 0u : a.olen ? a.olen[(uint64_t)s * a.m + i] : a.unit_bytes;
+    w.p[i] = reinterpret_cast<uint8_t*>(q);
+    w.plen[i] = q ? (l < a.unit_bytes ? l : a.unit_bytes) : 0u;
+  }
+  MfmaCode<KH, MH> code;
+  code.template load<kBlock>(a.coeff, w.code);
+  __syncthreads();
+  const uint32_t lane = t & 63u, half = lane >> 5;
+  for (uint32_t step = s0 + __builtin_amdgcn_readfirstlane(t >> 6); step < s1; step += kWaves) {
+    const uint32_t lo = step * kCoreStep, off = lo + (lane & 31u) * 16u;
+    uint4 x[KT][4];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < mfma_words(KH, kt); ++i) {
+        const uint32_t j = 8 * kt + 2 * i + half;
+        const uint32_t l = w.len[j];
+        x[kt][i] = load_any(l > lo ? clip_address(w.d[j], off, l) : g_zeros);
+      }
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int i = 0; i < mfma_words(KH, kt); ++i) {
+        const uint32_t j = 8 * kt + 2 * i + half;
+        const uint32_t l = w.len[j];
+        if (l > lo && l < lo + kCoreStep)
+          x[kt][i] = l >= 16u ? clip_chunk(x[kt][i], off, l)
+                     : off < l ? load_short(w.d[j], l) : x[kt][i];
+      }
+    uint32_t c[KT][4][4];
+    mfma_columns<KH, false>(c, x);
+    uint4 out[MT][2];
+    mfma_matvec16<KH, MH, PAIR>(out, c, code);
+    asm volatile("" ::: "memory");   // the descriptors stay in LDS
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int q = 0; q < mfma_outs(MH, mt); ++q) {
+        const uint32_t o = 4 * mt + 2 * q + half;
+        store_clip(w.p[o], off, w.plen[o], out[mt][q]);
+      }
+  }
+}
+
+template <int KH, int MH>
+int launch_core(const uint8_t* coeff, int k, int m, const uint64_t* dptr, const uint32_t* dlen,
+                const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,
+                uint32_t unit_bytes, hipStream_t st) {
+  BatchCoreArgs a;
+  a.dptr = dptr;
+  a.dlen = dlen;
+  a.pptr = pptr;
+  a.olen = olen;
+  a.coeff = mfma_coeff(coeff, k, m);
+  a.k = k;
+  a.m = m;
+  a.unit_bytes = unit_bytes;
+  a.steps_per_unit = (unit_bytes + kCoreStep - 1) / kCoreStep;
+  // Spans of span_bytes per workgroup, shorter where fewer than 2048
+  // workgroups would be left, a step per wave at least.
+  const uint64_t total = (uint64_t)n_stripes * a.steps_per_unit;
+  uint64_t spb = span_bytes(unit_bytes) / kCoreStep;
+  if (total / spb < 2048) spb = total / 2048;
+  if (spb < kBlock / 64) spb = kBlock / 64;
+  if (spb > a.steps_per_unit) spb = a.steps_per_unit;
+  a.steps_per_block = (uint32_t)spb;
+  a.blocks_per_unit = (a.steps_per_unit + a.steps_per_block - 1) / a.steps_per_block;
+  a.by_blocks = make_fastdiv(a.blocks_per_unit);
+  const uint64_t blocks = (uint64_t)n_stripes * a.blocks_per_unit;
+  if (blocks > 0x7fffffffull) return EC_ERANGE;
+  bool pair = true;
+  if constexpr (KH == EC_MAX_K / 4) pair = mfma_pair_ok(coeff, k, m);
+  const dim3 grid((unsigned)blocks), block(kBlock);
+  if (pair)
+    hipLaunchKernelGGL((batched_core_kernel<KH, MH, true>), grid, block, 0, st, a);
+  else if constexpr (KH == EC_MAX_K / 4)
+    hipLaunchKernelGGL((batched_core_kernel<KH, MH, false>), grid, block, 0, st, a);
+  return hip_status();
+}
+
+constexpr uint64_t kBatchTableBytes = 16u << 20;   // of each position
+
+using CoreFn = int (*)(const uint8_t*, int, int, const uint64_t*, const uint32_t*,
+                       const uint64_t*, const uint32_t*, uint32_t, uint32_t, hipStream_t);
+template <int KH, int... Ms>
+constexpr auto core_row(std::integer_sequence<int, Ms...>) {
+  return std::array<CoreFn, sizeof...(Ms)>{&launch_core<KH, Ms + 1>...};
+}
+template <int... Ks>
+constexpr auto core_table(std::integer_sequence<int, Ks...>) {
+  return std::array<std::array<CoreFn, EC_MAX_M / 2>, sizeof...(Ks)>{
+      core_row<Ks + 1>(std::make_integer_sequence<int, EC_MAX_M / 2>{})...};
+}
+const auto kCoreTable = core_table(std::make_integer_sequence<int, EC_MAX_K / 4>{});
+
 // The update's launch shape (update_kernel in ec_update.h): lanes per
 // workgroup, 16-byte chunks per lane, and log2 of the interleaved slices of
 // the grid (0: launch order).  Measured on MI355X for config 5's 1 % update
@@ -302,6 +449,16 @@ int batched_wide(int m, const uint8_t* coeff, int k, const uint64_t* dptr, const
                  const uint64_t* optr, const uint64_t* pptr, const uint32_t* olen,
                  uint32_t n_stripes, uint32_t unit_bytes, bool update, hipStream_t st) {
   if (m < 1 || m > EC_MAX_M || k < 1 || k > EC_MAX_K) return EC_ERANGE;
+  // The tables where they clearly cost less (table_cost against core_cost, see
+  // ec_mfma.h) and enough stripes run to be bound by it (us, tables / matrix
+  // cores, 100 tensors in 64 KiB units: RS(10,6) 293 / 316, RS(20,2) 176 / 192;
+  // RS(6,8) 406 / 394, RS(20,4) 216 / 208, RS(24,8) 341 / 243, RS(32,16) 588 /
+  // 390; RS(10,6) over 5 MB of 16 KiB stripes 25.0 / 21.2).
+  const bool tables = (uint64_t)n_stripes * unit_bytes > kBatchTableBytes &&
+                      4 * table_cost(k, m) <= 3 * core_cost(k, m);
+  if (!update && !tables)
+    return kCoreTable[(k - 1) / 4][(m - 1) / 2](coeff, k, m, dptr, dlen, pptr, olen, n_stripes,
+                                                unit_bytes, st);
   return kBatchWideTable[m - 1](coeff, k, dptr, dlen, optr, pptr, olen, n_stripes, unit_bytes,
                                 update, st);
 }

@@ -201,3 +201,40 @@ def test_units_of_every_length_around_the_chunk(pkg, dev, k, m, unit, skew):
     torch.cuda.synchronize()
     now = [t.cpu().numpy() for t in tensors]
     assert np.array_equal(parity.cpu().numpy(), expected(now))
+
+
+@pytest.mark.parametrize("k,m,unit,n", [(10, 6, 16 << 10, 17 << 20), (20, 2, 64 << 10, 17 << 20),
+                                        (24, 8, 4096, 1 << 20), (32, 16, 512, 100_000),
+                                        (32, 3, 1536, 50_000)])
+def test_batched_wide_routes(pkg, dev, k, m, unit, n):
+    """Both sides of the rule between the tables and the matrix cores (16 MiB of
+    each position), odd numbers of 512-byte steps, and the deepest code."""
+    rng = np.random.default_rng([k, m])
+    sizes = [n * k * 3 // 5 + 7, n * k * 2 // 5 + 1, 333]
+    flat = torch.randint(0, 256, (sum(sizes) + 64,), dtype=torch.uint8, device=dev,
+                         generator=torch.Generator(device=dev).manual_seed(k))
+    starts = np.cumsum([0] + [-(-s // 16) * 16 for s in sizes[:-1]])
+    tensors = [flat[int(a): int(a) + s] for a, s in zip(starts, sizes)]
+    lay = pkg.StripeLayout(tensors, k, m, unit)
+    parity = lay.encode()
+    # sampled stripes against the scalar oracle
+    pick = sorted({0, lay.n_stripes - 1, *(int(x) for x in rng.integers(0, lay.n_stripes, 6))})
+    grid, ln = [], []
+    for s in pick:
+        row = [lay.unit_view(s * k + j).cpu().numpy() if s * k + j < lay.n_units else None
+               for j in range(k)]
+        grid.append(row)
+        ln.append([0 if r is None else r.size for r in row])
+    want = oracle.encode_batched(lay.coeff, grid, np.array(ln, np.uint32), unit)
+    assert np.array_equal(parity[pick].cpu().numpy(), want)
+    # and every stripe back from the parity
+    before, par = flat.clone(), parity.clone()
+    lost = sorted(int(x) for x in rng.choice(k + m, min(m, 5), replace=False))
+    for p in lost:
+        if p >= k:
+            parity[:, p - k].fill_(1)
+    gone = [lay.unit_view(s * k + p) for p in lost if p < k for s in range(lay.n_stripes)
+            if s * k + p < lay.n_units]
+    torch._foreach_zero_(gone)
+    lay.decode(parity, lost)
+    assert torch.equal(flat, before) and torch.equal(parity, par)
