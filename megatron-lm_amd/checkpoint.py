@@ -200,7 +200,7 @@ class GpuSliceCodec:
     fits (see ``snapshot``) and stages it with ``ec_stage_stripes_to_host``;
     otherwise the work goes in chunks of stripes of at most ``chunk_bytes``,
     double-buffered on the device and in pinned host memory: 2 * chunk_bytes
-    of extra HBM and of page-locked memory.  ``decode`` likewise takes one
+    of extra HBM and at most 128 MiB of page-locked memory (``_pinned_bytes``).  ``decode`` likewise takes one
     (k, stripes, unit_bytes) block when it fits, else chunks, and moves the
     slices up with ``ec_stage_to_device``.
 

@@ -1,6 +1,7 @@
 // ec_update.hip — ec_parity_update (update_kernel of ec_update.h for
 // k <= 16, m <= 4) and the batched kernels for wide codes
-// (batched_wide_kernel, update_wide_kernel: k at run time, up to
+// (batched_core_kernel on the matrix cores; batched_wide_kernel and
+// update_wide_kernel on permute tables, k at run time; up to
 // EC_MAX_K x EC_MAX_M), which ec_batched.hip and ec_batched_copy.hip reach
 // through batched_wide().
 #include <hip/hip_runtime.h>
