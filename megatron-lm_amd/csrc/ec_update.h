@@ -159,9 +159,11 @@ __global__ void __launch_bounds__(B) update_kernel(const UpdateArgs<K, M> a) {
 #pragma unroll
       for (int i = 0; i < M; ++i) pv[i] = load_any(p[i] + off);
       uint32_t acc[M][4] = {};
-      // A loop over the descriptors in memory, four units' loads in flight at a
-      // time: few tiles, so kept small and below the vector path's registers.
-      constexpr int G = K < 4 ? K : 4;
+      // A loop over the descriptors in memory, two units' loads in flight at a
+      // time: few tiles, so kept within the vector path's registers (four units
+      // and tables read ahead took RS(12,4) to 150, three waves per SIMD; 125 and
+      // four now).
+      constexpr int G = K < 2 ? K : 2;
 #pragma unroll 1
       for (int j0 = 0; j0 < K; j0 += G) {
         const uint8_t* n[G];
@@ -198,6 +200,7 @@ __global__ void __launch_bounds__(B) update_kernel(const UpdateArgs<K, M> a) {
           for (int dd = 0; dd < 4; ++dd) f[dd] = fields(word(dl, dd));
 #pragma unroll
           for (int i = 0; i < M; ++i) {
+            asm volatile("" ::: "memory");   // each table right before its uses
             const PermTab tj = tab[i][j0 + g];
 #pragma unroll
             for (int dd = 0; dd < 4; ++dd) acc[i][dd] = mac1(acc[i][dd], tj, f[dd]);
