@@ -296,9 +296,10 @@ class GpuSliceCodec:
         a half is a 32nd of the total, between 4 and 64 MiB (a page of each of
         ``rows`` rows at least), within 2 * ``chunk_bytes`` in all.  The first
         half's transfer (upwards: its fill) and the last one's host copy
-        overlap nothing, so halves of 1 GiB left a 1.4 GB block with two steps
-        one after the other: saving a 1.04 GB state (RS(12,4), 64 KiB units)
-        took 31.6 ms with them, 22.9 with these, of which the link takes 22.
+        overlap nothing, so halves of 1 GiB left a block of 1.07 GB with two
+        steps one after the other: saving a 0.80 GB state (RS(12,4), 64 KiB
+        units) took 32.0 ms with them, 21.0 with these; the link alone takes
+        about 19.
         A 4 MiB half is 74 us of the link, more than a transfer's start and the
         copying threads' cost."""
         half = max(4 << 20, min(64 << 20, total // 32), 4096 * rows)
