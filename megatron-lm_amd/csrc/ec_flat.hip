@@ -306,7 +306,9 @@ __global__ void __launch_bounds__(kXorBlock) any_xor_kernel(const AnyXorArgs<K> 
   }
 }
 
-// Shards of less than 16 bytes: one lane per byte, any k and m.
+// Shards of less than 16 bytes, any k and m: a lane per byte and output, all
+// in one workgroup.  Every output is coded before any is stored, since an
+// output may lie over an input.
 struct TinyArgs {
   const uint8_t* data[EC_MAX_K];
   uint8_t* out[EC_MAX_M];
@@ -315,14 +317,17 @@ struct TinyArgs {
   int k, m;
 };
 
-__global__ void __launch_bounds__(64) tiny_kernel(const TinyArgs a) {
+constexpr int kTinyBlock = 16 * EC_MAX_M;
+
+__global__ void __launch_bounds__(kTinyBlock) tiny_kernel(const TinyArgs a) {
   const uint32_t b = threadIdx.x & 15u;
-  if (b >= a.n) return;
-  for (int i = threadIdx.x >> 4; i < a.m; i += 4) {
-    uint8_t acc = 0;
+  const int i = threadIdx.x >> 4;
+  const bool mine = b < a.n && i < a.m;
+  uint8_t acc = 0;
+  if (mine)
     for (int j = 0; j < a.k; ++j) acc ^= dev_gf_mul(a.coeff[i * a.k + j], gptr(a.data[j])[b]);
-    gptr(a.out[i])[b] = acc;
-  }
+  __syncthreads();
+  if (mine) gptr(a.out[i])[b] = acc;
 }
 
 // ------------------------------------------------------------ table kernel --
@@ -821,7 +826,7 @@ int launch_tiny(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uin
   a.n = (uint32_t)n;
   a.k = k;
   a.m = m;
-  hipLaunchKernelGGL(tiny_kernel, dim3(1), dim3(64), 0, st, a);
+  hipLaunchKernelGGL(tiny_kernel, dim3(1), dim3(kTinyBlock), 0, st, a);
   return hip_status();
 }
 

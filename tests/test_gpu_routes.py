@@ -108,6 +108,23 @@ def test_output_over_an_input(pkg, dev, k, m, offset):
         assert np.array_equal(shards[i].cpu().numpy(), want[i])
 
 
+@pytest.mark.parametrize("k,m", [(4, 4), (5, 5), (10, 6), (24, 8), (32, 16)])
+def test_output_over_an_input_of_a_few_bytes(pkg, dev, k, m):
+    """The same below one chunk, where a lane codes several outputs: none may be
+    stored while another is still to be read from what it overwrites."""
+    for n in (1, 7, 15):
+        rng = np.random.default_rng([k, n])
+        host = [rng.integers(0, 256, n, dtype=np.uint8) for _ in range(k)]
+        shards, _ = _carve(dev, host, [(3 * j + 1) % 16 for j in range(k)])
+        C = oracle.cauchy(k, m)
+        pkg.matvec(C, shards, out=shards[:m])
+        want = [np.empty(n, np.uint8) for _ in range(m)]
+        oracle.fast_rs_encode(C, host, want)
+        torch.cuda.synchronize()
+        for i in range(m):
+            assert np.array_equal(shards[i].cpu().numpy(), want[i]), f"n={n} output {i}"
+
+
 @pytest.mark.parametrize("k", [1, 2, 5, 16, 17, 32])
 def test_xor_any_shards(pkg, dev, k):
     for n in [1, 16, 17, 1023, 1040, 70_001]:
