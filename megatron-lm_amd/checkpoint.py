@@ -202,7 +202,8 @@ class GpuSliceCodec:
     double-buffered on the device and in pinned host memory: 2 * chunk_bytes
     of extra HBM and at most 128 MiB of page-locked memory (``_pinned_bytes``).  ``decode`` likewise takes one
     (k, stripes, unit_bytes) block when it fits, else chunks, and moves the
-    slices up with ``ec_stage_to_device``.
+    slices up with ``ec_stage_to_device`` through at most 512 MiB of page-locked
+    memory (``_pinned_load_bytes``).
 
     The slices own their host array (they are views of it): the codec keeps
     no reference to an array it handed out, so nothing the caller holds,
@@ -291,19 +292,40 @@ class GpuSliceCodec:
         with self._host_lock:
             self._free = base
 
-    def _pinned_bytes(self, total: int, rows: int = 1) -> int:
-        """Bytes of pinned memory to stage ``total`` bytes through, two halves:
-        a half is a 32nd of the total, between 4 and 64 MiB (a page of each of
-        ``rows`` rows at least), within 2 * ``chunk_bytes`` in all.  The first
-        half's transfer (upwards: its fill) and the last one's host copy
-        overlap nothing, so halves of 1 GiB left a block of 1.07 GB with two
-        steps one after the other: saving a 0.80 GB state (RS(12,4), 64 KiB
-        units) took 32.0 ms with them, 21.0 with these; the link alone takes
-        about 19.
-        A 4 MiB half is 74 us of the link, more than a transfer's start and the
-        copying threads' cost."""
-        half = max(4 << 20, min(64 << 20, total // 32), 4096 * rows)
+    def _pinned_bytes(self, total: int) -> int:
+        """Bytes of pinned memory to stage a block of ``total`` bytes down
+        through, two halves: a half is a 32nd of the total, between 4 and
+        64 MiB, within 2 * ``chunk_bytes`` in all.  The first half's transfer
+        and the last one's host copy overlap nothing, so halves of 1 GiB left
+        a block of 1.07 GB with two steps one after the other: saving a 0.80 GB
+        state (RS(12,4), 64 KiB units) took 32.0 ms with them, 21.0 with these;
+        the link alone takes about 19.  A half goes down in one transfer: 4 MiB
+        are 74 us of the link, more than a transfer's start and the copying
+        threads' cost."""
+        half = max(4 << 20, min(64 << 20, total // 32))
         return min(2 * self.chunk_bytes, 2 * total, 2 * half)
+
+    def _pinned_load_bytes(self, row: int, rows: int) -> int:
+        """Bytes of pinned memory to stage ``rows`` rows of ``row`` bytes up
+        through, two halves.  A half goes up in one transfer per row and is
+        filled by threads started for it, so it must be long for both: 32 MiB or
+        4 MiB of every row, and an eighth of the load, up to 256 MiB, where that
+        is more (within 2 * ``chunk_bytes`` in all).  Loads of less than two such
+        halves go up in one piece, longer ones in equal pieces.  Measured on
+        MI355X (ms a load, in one piece / halves of 4, 32, 64, 128 and 256 MiB;
+        *: as chosen here):
+          k = 4,  100 MiB   3.47 / 4.35  3.05*  3.25  3.45
+          k = 12,  20 MiB   1.27* / 1.83
+          k = 12, 100 MiB   3.47 / 5.99  3.39*  3.37  3.49
+          k = 24, 100 MiB   3.74* / 9.16  3.99  3.73  3.72
+          k = 32, 100 MiB   3.80* / 10.83  4.34  3.86
+          k = 12, 1000 MiB  28.8 / 52.0  25.1  23.4  23.3*  23.7
+          k = 32, 1000 MiB  28.9 / 98.6  31.6  26.7  24.4*  24.1
+          k = 24, 4000 MiB  92.9 /   -  113.0  99.2  91.8  87.7*"""
+        total = row * rows
+        half = max(32 << 20, rows * (4 << 20), min(256 << 20, total // 8))
+        piece = -(-row // max(1, total // half))
+        return min(2 * self.chunk_bytes, 2 * rows * (-(-piece // 4096) * 4096))
 
     def _chunk_stripes(self, n_stripes: int, rows: int) -> int:
         return max(1, min(n_stripes, self.chunk_bytes // (rows * self.unit_bytes)))
@@ -640,7 +662,7 @@ class GpuSliceCodec:
                     C = self._chunk_stripes(S, k)
             for bf in bufs:
                 bf.record_stream(copy)
-            pinned = torch.empty(self._pinned_bytes(k * C * U, k), dtype=torch.uint8,
+            pinned = torch.empty(self._pinned_load_bytes(C * U, k), dtype=torch.uint8,
                                  pin_memory=True)
             # Every descriptor array is uploaded once, stripe-major, so that a
             # chunk's descriptors are a contiguous slice (a pointer offset).

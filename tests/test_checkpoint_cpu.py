@@ -161,6 +161,26 @@ def test_ec_nccl_group_without_gloo_is_refused(monkeypatch):
         st.comm_group()
 
 
+@pytest.mark.parametrize("k", [1, 4, 12, 24, 32])
+def test_load_halves_carry_whole_loads_or_megabytes_per_row(pkg, k):
+    """A half of the upload's pinned memory costs one transfer per row and a set
+    of host threads: it holds the whole load, or 4 MiB and more of every row."""
+    from megatron_lm_amd.checkpoint import GpuSliceCodec
+    codec = GpuSliceCodec(k, 1, 4096)
+    for total in [1 << 20, 5 << 20, 20 << 20, 70 << 20, 100 << 20, 250 << 20, 1 << 30, 8 << 30]:
+        row = -(-total // k // 4096) * 4096
+        half = codec._pinned_load_bytes(row, k) // 2
+        width = half // k                  # bytes of a row in a half
+        least = max(32 << 20, k * (4 << 20))
+        assert half >= min(row * k, least) and half < max(2 * least, 512 << 20)
+        tail = row % width                 # no short last piece
+        assert tail == 0 or tail * 8 >= width * 7
+    for row in (16, 4112, (3 << 20) + 16):   # units that are not whole pages: one piece all the same
+        assert codec._pinned_load_bytes(row, k) // 2 // k >= row
+    small = GpuSliceCodec(k, 1, 4096, chunk_bytes=1 << 20)
+    assert small._pinned_load_bytes(1 << 30, k) == 2 << 20
+
+
 def test_slice_host_arrays_are_reused_only_after_release():
     """GpuSliceCodec's host arrays (host side only, no GPU): the slices own
     their array and the codec keeps no reference to one it handed out, so a
