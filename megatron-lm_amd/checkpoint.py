@@ -294,15 +294,21 @@ class GpuSliceCodec:
 
     def _pinned_bytes(self, total: int) -> int:
         """Bytes of pinned memory to stage a block of ``total`` bytes down
-        through, two halves: a half is a 32nd of the total, between 4 and
+        through, two halves: a half is a 32nd of the total, between 16 and
         64 MiB, within 2 * ``chunk_bytes`` in all.  The first half's transfer
         and the last one's host copy overlap nothing, so halves of 1 GiB left
         a block of 1.07 GB with two steps one after the other: saving a 0.80 GB
         state (RS(12,4), 64 KiB units) took 32.0 ms with them, 21.0 with these;
-        the link alone takes about 19.  A half goes down in one transfer: 4 MiB
-        are 74 us of the link, more than a transfer's start and the copying
-        threads' cost."""
-        half = max(4 << 20, min(64 << 20, total // 32))
+        the link alone takes about 19.  A half goes down in one transfer, but
+        its copying threads are started for it, about as long as 4 MiB take on
+        the link.  Measured on MI355X (RS(12,4), ms a save, in one piece /
+        halves of 4, 8, 16, 32 and 64 MiB):
+           10 MiB  0.71 / 0.71  0.74
+           20 MiB  1.19 / 1.29  1.10  1.05
+           50 MiB  2.34 / 2.35  1.80  1.87  2.03  2.38
+          200 MiB  8.64 / 9.27  6.40  6.06  6.15  6.45
+         1000 MiB  33.2 / 42.0  29.2  27.2  26.9  27.2"""
+        half = max(16 << 20, min(64 << 20, total // 32))
         return min(2 * self.chunk_bytes, 2 * total, 2 * half)
 
     def _pinned_load_bytes(self, row: int, rows: int) -> int:

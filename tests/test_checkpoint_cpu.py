@@ -181,6 +181,19 @@ def test_load_halves_carry_whole_loads_or_megabytes_per_row(pkg, k):
     assert small._pinned_load_bytes(1 << 30, k) == 2 << 20
 
 
+def test_save_halves_carry_small_saves_whole():
+    """A half of the download's pinned memory costs a set of host threads: a
+    block of up to 16 MiB goes down in one, larger ones in halves of 16 to 64."""
+    import __graft_entry__
+    __graft_entry__.load_package()
+    from megatron_lm_amd.checkpoint import GpuSliceCodec
+    codec = GpuSliceCodec(12, 4, 65536)
+    for total in (65536, 5 << 20, 16 << 20):
+        assert codec._pinned_bytes(total) == 2 * total
+    for total in (20 << 20, 100 << 20, 1 << 30, 20 << 30):
+        assert 16 << 20 <= codec._pinned_bytes(total) // 2 <= 64 << 20
+
+
 def test_slice_host_arrays_are_reused_only_after_release():
     """GpuSliceCodec's host arrays (host side only, no GPU): the slices own
     their array and the codec keeps no reference to one it handed out, so a
