@@ -42,6 +42,7 @@
 #include "ec_mi355.h"
 #include "fastdiv.h"
 #include "gf256.h"
+#include "routes.h"
 
 namespace ec {
 
@@ -59,8 +60,6 @@ int batched_wide(int m, const uint8_t* coeff, int k, const uint64_t* dptr, const
 namespace {
 
 constexpr int kBlock = 256;     // lanes per workgroup (4 wavefronts)
-constexpr int kFastMaxK = 16;   // template-instantiated shard counts
-constexpr int kFastMaxM = 4;
 // Bytes of each unit a workgroup of the batched kernels for wide codes
 // (batched_wide_kernel, 4 KiB tiles) walks: 8 KiB for units up to 256 KiB,
 // 16 KiB above.  Measured on MI355X for the fixed-size batched kernel when it
@@ -349,7 +348,7 @@ constexpr int kWidePair() {
 }
 
 // 16 bytes at base + off, where off is a multiple of 16 and base may have any
-// alignment (uniform: it depends on the shard only), for the table kernel:
+// alignment (uniform: it depends on the unit only), for the parity update:
 // the aligned dwordx4 load, or one at the unaligned address.
 __device__ __forceinline__ uint4 load_realign(const uint8_t* base, uint64_t off) {
   if ((reinterpret_cast<uintptr_t>(base) & 15u) == 0) return load_stream(base + off);
@@ -522,8 +521,6 @@ __device__ __forceinline__ uint32_t span_of(const SpanGrid& g) {
   const uint32_t b = blockIdx.x;
   return (b & ((1u << g.slice_shift) - 1u)) * g.slice_spans + (b >> g.slice_shift);
 }
-
-inline bool fast_shape(int k, int m) { return k <= kFastMaxK && m <= kFastMaxM; }
 
 inline int check_batch(const uint8_t* coeff, int k, int m, const void* a, const void* b,
                 const void* c, uint32_t unit_bytes) {

@@ -332,20 +332,22 @@ __global__ void __launch_bounds__(kTinyBlock) tiny_kernel(const TinyArgs a) {
 
 // ------------------------------------------------------------ table kernel --
 // Codes past the unrolled kernels for which the permute tables cost less than
-// the matrix cores (see matvec), on whole chunks at aligned addresses: see
+// the matrix cores (flat_route in routes.h), any size and alignment: see
 // kWideGroup in ec_device.h.
 struct TableArgs {
   const uint8_t* data[EC_MAX_K];
   uint8_t* out[EC_MAX_M];
   uint8_t coeff[EC_MAX_M * EC_MAX_K];  // row-major m x k
-  uint64_t n16;
+  Frame f;
   int k;
 };
 
 // 128-lane workgroups in launch order.  Measured on MI355X (HBM traffic,
 // TB/s, 64 MiB shards): RS(17,1) 6.1, RS(20,2) 5.8, RS(6,12) 5.5, RS(10,12)
 // 4.6; 256-lane workgroups that streamed each shard at two places half a shard
-// apart were 1-6 % slower.
+// apart were 1-6 % slower.  Shards of 64 MiB + 5 B at the rate of whole chunks
+// (us, on the matrix cores before / here): RS(17,1) 216 / 196, RS(6,9) 203 / 178,
+// RS(10,10) 326 / 277, RS(4,16) 283 / 241, XOR of 32 381 / 362.
 constexpr int kTableBlock = 128;
 
 template <int M>
@@ -354,15 +356,18 @@ __global__ void __launch_bounds__(kTableBlock) table_kernel(const TableArgs a) {
   const int k = a.k;
   for (int t = threadIdx.x; t < M * k; t += kTableBlock) tab[t] = dev_perm_tab(a.coeff[t]);
   __syncthreads();
-  const uint64_t stride = (uint64_t)gridDim.x * kTableBlock;
-  for (uint64_t idx = (uint64_t)blockIdx.x * kTableBlock + threadIdx.x;
-       idx < a.n16; idx += stride) {
+  const uint64_t steps = edge_steps(a.f) + (a.f.n16 + kTableBlock - 1) / kTableBlock;
+  for (uint64_t step = blockIdx.x; step < steps; step += gridDim.x) {
+    const Step s = step_of(a.f, step, kTableBlock);
+    if (threadIdx.x >= s.chunks) continue;
+    uint32_t lane = threadIdx.x * 16u;
+    asm volatile("" : "+v"(lane));   // no address is kept over the steps
     uint32_t acc[M][4] = {};
     for (int j0 = 0; j0 < k; j0 += kWideGroup) {
       uint4 x[kWideGroup];
 #pragma unroll
       for (int g = 0; g < kWideGroup; ++g)
-        x[g] = j0 + g < k ? load_realign(a.data[j0 + g], idx * 16) : make_uint4(0, 0, 0, 0);
+        x[g] = j0 + g < k ? load_any(a.data[j0 + g] + s.at + lane) : make_uint4(0, 0, 0, 0);
 #pragma unroll
       for (int g = 0; g < kWideGroup; g += kWidePair<M>()) {
         if (j0 + g >= k) break;
@@ -399,9 +404,16 @@ __global__ void __launch_bounds__(kTableBlock) table_kernel(const TableArgs a) {
         }
       }
     }
+    pin_products(acc);
+    if (whole(s)) {
 #pragma unroll
-    for (int i = 0; i < M; ++i)
-      store_stream(a.out[i] + idx * 16, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
+      for (int i = 0; i < M; ++i)
+        store_any(a.out[i] + s.at + lane, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
+    } else {
+#pragma unroll
+      for (int i = 0; i < M; ++i)
+        store_edge(a.out[i] + s.at, s, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
+    }
   }
 }
 
@@ -677,15 +689,16 @@ int launch_wide(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uin
 
 template <int M>
 int launch_table(const uint8_t* coeff, int k, const uint8_t* const* d, uint8_t* const* o,
-                 uint64_t n16, hipStream_t st) {
+                 const Frame& f, hipStream_t st) {
   TableArgs a;
   for (int j = 0; j < k; ++j) a.data[j] = d[j];
   for (int i = 0; i < M; ++i) a.out[i] = o[i];
   for (int t = 0; t < M * k; ++t) a.coeff[t] = coeff[t];
-  a.n16 = n16;
+  a.f = f;
   a.k = k;
-  hipLaunchKernelGGL((table_kernel<M>), dim3(grid_of(n16, kTableBlock)), dim3(kTableBlock), 0, st,
-                     a);
+  const uint64_t steps = frame_steps(f, kTableBlock);
+  hipLaunchKernelGGL((table_kernel<M>), dim3((unsigned)(steps < kMaxGrid ? steps : kMaxGrid)),
+                     dim3(kTableBlock), 0, st, a);
   return hip_status();
 }
 
@@ -727,7 +740,6 @@ template <int K, int... Ms>
 constexpr auto any_row(std::integer_sequence<int, Ms...>) {
   return std::array<AnyFn, sizeof...(Ms)>{&launch_any<K, Ms + 1>...};
 }
-constexpr int kAnyMaxM = 8, kAnyDeepMaxK = 12;   // M > kFastMaxM: k <= kAnyDeepMaxK
 template <int K>
 constexpr auto any_row_of() {
   constexpr int kMs = K <= kAnyDeepMaxK ? kAnyMaxM : kFastMaxM;
@@ -744,7 +756,7 @@ template <int... Ks>
 constexpr auto any_xor_table(std::integer_sequence<int, Ks...>) {
   return std::array<AnyXorFn, sizeof...(Ks)>{&launch_any_xor<Ks + 1>...};
 }
-using TableFn = int (*)(const uint8_t*, int, const uint8_t* const*, uint8_t* const*, uint64_t,
+using TableFn = int (*)(const uint8_t*, int, const uint8_t* const*, uint8_t* const*, const Frame&,
                         hipStream_t);
 template <int... Ms>
 constexpr auto table_table(std::integer_sequence<int, Ms...>) {
@@ -801,22 +813,6 @@ inline Frame frame_of(uint8_t* const* o, int m, uint64_t nbytes) {
   return f;
 }
 
-// Whether the permute tables take fewer cycles than the matrix cores for a
-// code past the unrolled kernels.  Both kernels over 64 MiB shards (HBM traffic, TB/s, tables /
-// matrix cores; * any_kernel's tables): RS(17,1) 6.03 / 5.48, RS(6,9) 5.59 /
-// 4.91, RS(4,16) 5.43 / 4.75, RS(10,10) 4.73 / 4.07, RS(20,5) 5.14 / 4.82,
-// RS(10,6) 5.95* / 4.82, RS(5,5) 5.92* / 5.02, RS(12,8) 5.17* / 5.24, and past
-// the line RS(8,12) 4.92 / 5.40, RS(16,6) 4.87 / 5.55, RS(20,4) 5.60 / 6.04,
-// RS(16,8) 4.36 / 5.55, RS(24,8) 4.09 / 5.38, RS(32,16) 2.69 / 3.93.
-bool table_pays(int k, int m) { return table_cost(k, m) <= core_cost(k, m); }
-
-// Up to this shard size too few waves run to be bound by either's arithmetic
-// and the matrix cores' shorter chains win for every code (2 MiB shards, us,
-// tables / matrix cores: RS(20,2) 11.9 / 10.7, RS(6,12) 11.3 / 10.5, RS(17,1)
-// 9.9 / 9.6, RS(16,5) 14.1 / 12.2; 4 MiB: 19.1 / 21.3, 18.4 / 20.7, 17.0 /
-// 19.5, 22.6 / 23.3).
-constexpr uint64_t kTableMinBytes = 2u << 20;
-
 int launch_tiny(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uint8_t* const* o,
                 uint64_t n, hipStream_t st) {
   TinyArgs a;
@@ -840,17 +836,18 @@ int matvec(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uint8_t*
     if (!d[j]) return EC_EINVAL;
   for (int i = 0; i < m; ++i)
     if (!o[i]) return EC_EINVAL;
-  if (nbytes < 16) return launch_tiny(coeff, k, m, d, o, nbytes, st);
-  if (fast_shape(k, m)) {
-    if (nbytes % 16 == 0 && all_aligned(d, k) && all_aligned(o, m))
+  const bool aligned = nbytes % 16 == 0 && all_aligned(d, k) && all_aligned(o, m);
+  switch (flat_route(k, m, nbytes, aligned)) {
+    case FlatRoute::kTiny:
+      return launch_tiny(coeff, k, m, d, o, nbytes, st);
+    case FlatRoute::kAligned:
       return kRsTable[k - 1][m - 1](coeff, d, o, nbytes / 16, st);
-    return kAnyTable[k - 1][m - 1](coeff, d, o, frame_of(o, m, nbytes), st);
-  }
-  if (nbytes > kTableMinBytes && table_pays(k, m)) {
-    if (m <= kAnyMaxM && k <= kAnyDeepMaxK)
+    case FlatRoute::kAny:
       return kAnyTable[k - 1][m - 1](coeff, d, o, frame_of(o, m, nbytes), st);
-    if (nbytes % 16 == 0 && all_aligned(o, m))
-      return kTableTable[m - 1](coeff, k, d, o, nbytes / 16, st);
+    case FlatRoute::kTable:
+      return kTableTable[m - 1](coeff, k, d, o, frame_of(o, m, nbytes), st);
+    case FlatRoute::kWide:
+      break;
   }
   return wide_fn(k, m)(coeff, k, m, d, o, frame_of(o, m, nbytes), st);
 }

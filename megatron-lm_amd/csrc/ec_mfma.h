@@ -39,8 +39,6 @@ typedef float v16f32 __attribute__((ext_vector_type(16)));
 
 constexpr int kFmtFp4 = 4;         // operand format selector of f8f6f4: e2m1
 constexpr int kScaleOne = 127;     // E8M0 block scale 2^0
-constexpr int kMfmaShards = 8;     // shards per 64-deep K step (4 per lane half)
-constexpr int kMfmaOutputs = 4;    // parity shards per 32-row tile
 
 constexpr uint8_t cx_gf_mul(uint32_t a, uint32_t b) {
   uint32_t r = 0;
@@ -90,16 +88,6 @@ constexpr int mfma_groups(int kh) { return (kh + 1) / 2; }
 constexpr int mfma_tiles(int mh) { return (mh + 1) / 2; }
 constexpr int mfma_words(int kh, int kt) { return 2 * kt + 1 < kh ? 4 : 2; }   // i < this
 constexpr int mfma_outs(int mh, int mt) { return 2 * mt + 1 < mh ? 2 : 1; }     // s < this
-
-// What a code costs on the permute tables and on the matrix cores: SIMD cycles
-// per 512 byte columns, 4 per VALU op (1.125 k m + 1.25 k ops per column
-// against the transposes, expansions and bit selects here) and 32 per MFMA;
-// the two kinds measured about additive.
-inline int table_cost(int k, int m) { return 36 * k * m + 40 * k; }
-inline int core_cost(int k, int m) {
-  const int kt = (k + kMfmaShards - 1) / kMfmaShards, mt = (m + kMfmaOutputs - 1) / kMfmaOutputs;
-  return 512 * kt * mt + 448 * kt + 240 * ((m + 1) / 2);
-}
 
 // The coefficients as the kernels take them: m rows padded to 32 bytes, zeros
 // past k and m, each group of eight in the order of the lane halves (h, i).

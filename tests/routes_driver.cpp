@@ -1,0 +1,38 @@
+// Checks ec::flat_route (megatron-lm_amd/csrc/routes.h) over every shape: the
+// kernel of a code past the unrolled ones does not depend on whether its
+// shards are whole chunks at aligned addresses, and every route has a kernel
+// for the shapes that take it.  Built with g++.
+#include <cstdint>
+#include <cstdio>
+
+#include "routes.h"
+
+using ec::FlatRoute;
+
+int main() {
+  int bad = 0;
+  const uint64_t two = ec::kTableMinBytes;
+  const uint64_t sizes[] = {1, 15, 16, 4096, two, two + 1, 2 * two, 2 * two + 1, (64u << 20) + 5};
+  for (int k = 1; k <= EC_MAX_K; ++k)
+    for (int m = 1; m <= EC_MAX_M; ++m)
+      for (uint64_t n : sizes) {
+        const FlatRoute odd = ec::flat_route(k, m, n, false), even = ec::flat_route(k, m, n, true);
+        bool ok = false;
+        if (n < 16) ok = odd == FlatRoute::kTiny && even == odd;
+        else if (ec::fast_shape(k, m)) ok = odd == FlatRoute::kAny && even == FlatRoute::kAligned;
+        else if (even != odd) ok = false;
+        else if (odd == FlatRoute::kAny) ok = n > two && ec::any_shape(k, m) && ec::table_pays(k, m);
+        else if (odd == FlatRoute::kTable) ok = n > two && !ec::any_shape(k, m) && ec::table_pays(k, m);
+        else ok = odd == FlatRoute::kWide;
+        // single losses of wide codes and XOR of many shards: tables at any size past the small ones
+        if (m == 1 && k > ec::kFastMaxK && n > two) ok = ok && odd == FlatRoute::kTable;
+        if (!ok) {
+          std::printf("RS(%d,%d) over %llu bytes: route %d, aligned %d\n", k, m,
+                      (unsigned long long)n, (int)odd, (int)even);
+          ++bad;
+        }
+      }
+  if (bad) return 1;
+  std::printf("routes driver ok\n");
+  return 0;
+}

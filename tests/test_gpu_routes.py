@@ -73,6 +73,18 @@ def test_both_sides_of_the_table_rule(pkg, dev, k, m):
     _check(pkg, dev, k, m, (2 << 20) + 16, lambda j: 4 * j % 16, lambda i: 0)
 
 
+@pytest.mark.parametrize("k,m", [(17, 1), (20, 2), (17, 3), (13, 5), (32, 2), (6, 9), (10, 12),
+                                 (2, 16)])
+def test_table_codes_at_any_size_and_alignment(pkg, dev, k, m):
+    """table_kernel with both edges, one, or none, and outputs at their own
+    offsets: sizes just past the matrix cores' range."""
+    n = 4 << 20
+    _check(pkg, dev, k, m, n + 16, lambda j: 0, lambda i: 0)
+    _check(pkg, dev, k, m, n + 33, lambda j: 0, lambda i: 0)
+    _check(pkg, dev, k, m, n + 48, lambda j: 4 * j % 16, lambda i: 4)
+    _check(pkg, dev, k, m, n + 2047, lambda j: (5 * j + 3) % 16, lambda i: (7 * i + 1) % 16)
+
+
 @pytest.mark.parametrize("m", [1, 4, 7, 16])
 def test_sums_of_256_ones(pkg, dev, m):
     """32 equal coefficients whose bit matrix has a row of ones: on shards of
