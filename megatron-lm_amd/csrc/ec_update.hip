@@ -174,10 +174,16 @@ __global__ void __launch_bounds__(B) update_wide_kernel(const BatchWideArgs a) {
   for (uint32_t t = t0; t < t1; ++t) {
     const uint32_t off = t * kWideTile + threadIdx.x * 16u;
     if (off >= longest) continue;
-    uint32_t acc[M][4] = {};
-    uint4 pv[M];  // the parity does not depend on the delta: load it first
+    // The products go on top of the parity itself, loaded first: with registers
+    // of their own for both m = 16 took 200, two waves per SIMD instead of five
+    // (RS(32,16) 1 % update in 1 MiB units 147 us against 132).
+    uint32_t acc[M][4];
 #pragma unroll
-    for (int i = 0; i < M; ++i) pv[i] = load_any(w.p[i] + off);
+    for (int i = 0; i < M; ++i) {
+      const uint4 v = load_any(w.p[i] + off);
+#pragma unroll
+      for (int dd = 0; dd < 4; ++dd) acc[i][dd] = word(v, dd);
+    }
 #pragma unroll 1
     for (int j = 0; j < k; ++j) {
       if (w.d[j] == nullptr || off >= w.len[j]) continue;  // unchanged unit, or past its end
@@ -186,10 +192,10 @@ __global__ void __launch_bounds__(B) update_wide_kernel(const BatchWideArgs a) {
       wide_mac<M>(acc, make_uint4(vn.x ^ vo.x, vn.y ^ vo.y, vn.z ^ vo.z, vn.w ^ vo.w),
                   &w.tab[j], k);
     }
+    asm volatile("" ::: "memory");   // the addresses are read again
 #pragma unroll
     for (int i = 0; i < M; ++i)
-      store_any(w.p[i] + off, make_uint4(pv[i].x ^ acc[i][0], pv[i].y ^ acc[i][1],
-                                         pv[i].z ^ acc[i][2], pv[i].w ^ acc[i][3]));
+      store_any(w.p[i] + off, make_uint4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]));
   }
 }
 

@@ -54,3 +54,10 @@ def test_batched_tables_keep_their_waves(tmp_path):
     found = _kernels("ec_update", tmp_path)
     got = {name: _waves(found[name]) for name in WIDE_TABLES}
     assert all(got[name] >= least for name, least in WIDE_TABLES.items()), got
+
+
+def test_wide_updates_keep_their_waves(tmp_path):
+    found = _kernels("ec_update", tmp_path)
+    least = {1: 8, 4: 7, 6: 5, 8: 4, 9: 3, 12: 3, 14: 2, 16: 3}
+    got = {m: _waves(found[f"update_wide_kernel<{m},256>"]) for m in least}
+    assert all(got[m] >= least[m] for m in least), got
