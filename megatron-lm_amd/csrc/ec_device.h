@@ -453,14 +453,12 @@ __device__ __forceinline__ void pin_products(uint32_t (&acc)[M][4]) {
 
 inline int hip_status() { return hipGetLastError() == hipSuccess ? EC_OK : EC_EHIP; }
 
-constexpr uint64_t kMaxGrid = 1u << 24;   // workgroups of a flat launch; more work loops
-
 // Grid of a grid-stride kernel with `lanes` lanes per workgroup and one chunk
 // per lane: one workgroup per `lanes` chunks, up to 2^24 workgroups (shards
 // up to 16 GiB with 64 lanes are covered in one pass).
 inline unsigned grid_of(uint64_t n16, int lanes) {
   const uint64_t g = (n16 + (uint64_t)lanes - 1) / (uint64_t)lanes;
-  return (unsigned)(g < kMaxGrid ? (g ? g : 1) : kMaxGrid);
+  return (unsigned)(g < max_grid(lanes) ? (g ? g : 1) : max_grid(lanes));
 }
 
 // ----------------------------------------- grid order of batched launches --

@@ -627,7 +627,7 @@ int launch_any(const uint8_t* coeff, const uint8_t* const* d, uint8_t* const* o,
   a.f = f;
   constexpr int B = flat_block<K, M>();
   const uint64_t steps = frame_steps(f, B);
-  const unsigned grid = (unsigned)(steps < kMaxGrid ? steps : kMaxGrid);
+  const unsigned grid = (unsigned)(steps < max_grid(B) ? steps : max_grid(B));
   if (grid == steps)
     hipLaunchKernelGGL((any_kernel<K, M, false>), dim3(grid), dim3(B), 0, st, a);
   else if constexpr (M <= kFastMaxM)
@@ -644,8 +644,8 @@ int launch_any_xor(const uint8_t* const* d, uint8_t* o, const Frame& f, hipStrea
   a.out = o;
   a.f = f;
   const uint64_t steps = frame_steps(f, kXorBlock);
-  hipLaunchKernelGGL((any_xor_kernel<K>), dim3((unsigned)(steps < kMaxGrid ? steps : kMaxGrid)),
-                     dim3(kXorBlock), 0, st, a);
+  const uint64_t grid = steps < max_grid(kXorBlock) ? steps : max_grid(kXorBlock);
+  hipLaunchKernelGGL((any_xor_kernel<K>), dim3((unsigned)grid), dim3(kXorBlock), 0, st, a);
   return hip_status();
 }
 
@@ -669,7 +669,7 @@ int launch_wide(const uint8_t* coeff, int k, int m, const uint8_t* const* d, uin
   a.m = m;
   constexpr uint64_t kWaves = kWideBlock / 64;
   const uint64_t blocks = (frame_steps(f, kWideChunks) + kWaves - 1) / kWaves;
-  const uint64_t cap = MH <= 2 ? kMaxGrid : mfma_groups(KH) >= 3 ? kWideGridDeep : kWideGrid;
+  const uint64_t cap = MH <= 2 ? max_grid(kWideBlock) : mfma_groups(KH) >= 3 ? kWideGridDeep : kWideGrid;
   const dim3 grid((unsigned)(blocks < cap ? blocks : cap)), block(kWideBlock);
   bool pair = true;
   if constexpr (KH == EC_MAX_K / 4) pair = mfma_pair_ok(coeff, k, m);
@@ -697,8 +697,8 @@ int launch_table(const uint8_t* coeff, int k, const uint8_t* const* d, uint8_t* 
   a.f = f;
   a.k = k;
   const uint64_t steps = frame_steps(f, kTableBlock);
-  hipLaunchKernelGGL((table_kernel<M>), dim3((unsigned)(steps < kMaxGrid ? steps : kMaxGrid)),
-                     dim3(kTableBlock), 0, st, a);
+  const uint64_t grid = steps < max_grid(kTableBlock) ? steps : max_grid(kTableBlock);
+  hipLaunchKernelGGL((table_kernel<M>), dim3((unsigned)grid), dim3(kTableBlock), 0, st, a);
   return hip_status();
 }
 

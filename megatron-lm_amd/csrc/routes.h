@@ -81,4 +81,11 @@ constexpr FlatRoute flat_route(int k, int m, uint64_t nbytes, bool aligned) {
   return table_kernel_pays(k, m, nbytes) ? FlatRoute::kTable : FlatRoute::kWide;
 }
 
+// Workgroups of one launch at most; more work loops in the kernel.  HIP refuses
+// a grid of 2^32 lanes and more.
+constexpr uint64_t max_grid(uint64_t lanes) {
+  constexpr uint64_t kMax = 1u << 24;
+  return kMax * lanes < (1ull << 32) ? kMax : 0xffffffffull / lanes;
+}
+
 }  // namespace ec

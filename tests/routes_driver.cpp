@@ -32,6 +32,12 @@ int main() {
           ++bad;
         }
       }
+  for (uint64_t lanes = 64; lanes <= 1024; lanes += 64)   // HIP's limit, and one pass over 16 GiB
+    if (ec::max_grid(lanes) * lanes >= 1ull << 32 || ec::max_grid(lanes) * lanes < 1u << 30) {
+      std::printf("max_grid(%llu) = %llu\n", (unsigned long long)lanes,
+                  (unsigned long long)ec::max_grid(lanes));
+      ++bad;
+    }
   if (bad) return 1;
   std::printf("routes driver ok\n");
   return 0;

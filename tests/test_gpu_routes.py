@@ -153,6 +153,41 @@ def test_xor_any_shards(pkg, dev, k):
             assert (got[:base] == GUARD).all() and (got[base + n:] == GUARD).all()
 
 
+def _fill(n, dev, seed):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    return torch.empty(n, dtype=torch.uint8, device=dev).random_(0, 256, generator=g)
+
+
+def test_unaligned_kernels_past_the_grid_cap(pkg, dev):
+    """Shards of 16 GiB + 4141 B at an odd address: more chunks than one pass of
+    one-wavefront workgroups covers, with both edges."""
+    n = (16 << 30) + 4141
+    a, b = _fill(n + 16, dev, 21)[1: 1 + n], _fill(n + 16, dev, 22)[3: 3 + n]
+    want = torch.bitwise_xor(a, b)
+    x = pkg.xor_encode([a, b])
+    assert torch.equal(x, want)
+    x = pkg.matvec(np.ones((1, 2), np.uint8), [a, b])[0]
+    assert torch.equal(x, want)
+    del a, b, want, x
+    torch.cuda.empty_cache()
+
+
+def test_wide_kernel_past_the_grid_cap(pkg, dev):
+    """24 shards (one tensor) of 32 GiB + 4101 B through wide_narrow_kernel: more
+    than a grid of 256-lane workgroups may hold.  Each row's coefficients add up
+    to 1, so every output equals the tensor."""
+    n = (32 << 30) + 4101
+    a = _fill(n, dev, 23)
+    C = np.arange(1, 73, dtype=np.uint8).reshape(3, 24)
+    C[:, 0] ^= np.bitwise_xor.reduce(C, axis=1) ^ 1
+    outs = pkg.matvec(C, [a] * 24)
+    for o in outs:
+        assert all(torch.equal(o[i: i + (4 << 30)], a[i: i + (4 << 30)]) for i in range(0, n, 4 << 30))
+    del a, outs, o
+    torch.cuda.empty_cache()
+
+
 # ------------------------------------------------------- batched edge tiles --
 
 @pytest.mark.parametrize("k,m,unit", [(4, 2, 1024), (12, 4, 1040), (8, 2, 4096), (6, 3, 16),
