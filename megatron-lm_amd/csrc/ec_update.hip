@@ -318,15 +318,25 @@ int launch_core(const uint8_t* coeff, int k, int m, const uint64_t* dptr, const 
   a.steps_per_block = (uint32_t)spb;
   a.blocks_per_unit = (a.steps_per_unit + a.steps_per_block - 1) / a.steps_per_block;
   a.by_blocks = make_fastdiv(a.blocks_per_unit);
-  const uint64_t blocks = (uint64_t)n_stripes * a.blocks_per_unit;
-  if (blocks > 0x7fffffffull) return EC_ERANGE;
+  if ((uint64_t)n_stripes * a.blocks_per_unit > 0x7fffffffull) return EC_ERANGE;
   bool pair = true;
   if constexpr (KH == EC_MAX_K / 4) pair = mfma_pair_ok(coeff, k, m);
-  const dim3 grid((unsigned)blocks), block(kBlock);
-  if (pair)
-    hipLaunchKernelGGL((batched_core_kernel<KH, MH, true>), grid, block, 0, st, a);
-  else if constexpr (KH == EC_MAX_K / 4)
-    hipLaunchKernelGGL((batched_core_kernel<KH, MH, false>), grid, block, 0, st, a);
+  // As many launches as the grid's limit asks for (units of a few bytes: one
+  // launch holds 2^24 stripes).
+  const uint32_t most = (uint32_t)(max_grid(kBlock) / a.blocks_per_unit);
+  for (uint32_t left = n_stripes; left != 0;) {
+    const uint32_t n = left < most ? left : most;
+    const dim3 grid(n * a.blocks_per_unit), block(kBlock);
+    if (pair)
+      hipLaunchKernelGGL((batched_core_kernel<KH, MH, true>), grid, block, 0, st, a);
+    else if constexpr (KH == EC_MAX_K / 4)
+      hipLaunchKernelGGL((batched_core_kernel<KH, MH, false>), grid, block, 0, st, a);
+    left -= n;
+    a.dptr += (uint64_t)n * k;
+    a.dlen += (uint64_t)n * k;
+    a.pptr += (uint64_t)n * m;
+    if (a.olen) a.olen += (uint64_t)n * m;
+  }
   return hip_status();
 }
 

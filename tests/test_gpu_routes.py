@@ -302,3 +302,33 @@ def test_batched_wide_routes(pkg, dev, k, m, unit, n):
     torch._foreach_zero_(gone)
     lay.decode(parity, lost)
     assert torch.equal(flat, before) and torch.equal(parity, par)
+
+
+def test_batched_core_kernel_past_one_grid(pkg, dev):
+    """2^24 + 5 stripes of 16-byte units, more than a grid of 256-lane workgroups
+    may hold.  The units repeat every 1024 stripes, so each parity unit equals
+    that of the first 1024, which the scalar oracle checks."""
+    k, m, unit, n, period = 17, 4, 16, (1 << 24) + 5, 1024
+    arena = _fill(period * k * unit, dev, 31)
+    stripe = torch.arange(n, dtype=torch.int64, device=dev).remainder_(period)
+    dptr = torch.empty((n, k), dtype=torch.int64, device=dev)
+    for j in range(k):
+        torch.add(stripe * (k * unit), arena.data_ptr() + j * unit, out=dptr[:, j])
+    dlen = torch.full((n, k), unit, dtype=torch.int32, device=dev)
+    parity = torch.zeros((n, m, unit), dtype=torch.uint8, device=dev)
+    pptr = parity.data_ptr() + unit * torch.arange(n * m, dtype=torch.int64, device=dev)
+    C = oracle.cauchy(k, m)
+    lib = pkg._lib
+    lib.check(lib.lib().ec_encode_batched(
+        lib.u8ptr(C), k, m, dptr.data_ptr(), dlen.data_ptr(), pptr.data_ptr(), n, unit,
+        pkg.codec.stream_handle(torch.cuda.current_stream(), torch.device(dev))), "ec_encode_batched")
+    torch.cuda.synchronize()
+    first = parity[:period]
+    units = arena.cpu().numpy().reshape(period, k, unit)
+    want = oracle.encode_batched(C, [list(s) for s in units], np.full((period, k), unit, np.uint32), unit)
+    assert np.array_equal(first.cpu().numpy(), want)
+    for a in range(period, n, 1 << 20):
+        b = min(n, a + (1 << 20))
+        assert torch.equal(parity[a:b], first[stripe[a:b]])
+    del dptr, dlen, pptr, parity
+    torch.cuda.empty_cache()
