@@ -1163,8 +1163,8 @@ def test_shard_plan_outputs_held_for_a_launch_on_another_stream(pkg, dev):
 def test_flat_kernels_past_the_grid_cap(pkg, dev):
     """Shards of 16 GiB + 4 KiB + 48 B: more 16-byte chunks than the flat
     kernels' one-pass grid covers (2^24 one-wavefront workgroups), so the
-    grid-stride loop runs a second time for the last chunks, and a byte tail
-    follows.  XOR(2) and RS(2,1) with unit coefficients both equal a ^ b
+    grid-stride loop runs a second time for the last chunks; whole chunks at
+    aligned addresses, so rs_kernel and xor_kernel.  XOR(2) and RS(2,1) with unit coefficients both equal a ^ b
     (XOR's wave-uniform loop, RS(2,1)'s per-lane loop); RS(4,1) over
     [a, b, a, b] with coefficients (1, 1, 1, 0) equals b and RS(1,1) with
     coefficient 1 equals a (the wave-uniform loop of the two pass forms of

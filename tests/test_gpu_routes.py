@@ -43,8 +43,9 @@ def _check(pkg, dev, k, m, n, in_off, out_off, coeff=None, data=None, seed=0):
             f"RS({k},{m}) n={n} output {i}: bytes around it changed"
 
 
-# unrolled tables in registers / in LDS, any_kernel's five to eight outputs,
-# m <= 4 and k > 16, the deep codes with their bit matrix in registers / in LDS
+# unrolled tables in registers / in LDS, the matrix cores with five and more
+# outputs, with m <= 4 and k > 16, and the deep codes with their bit matrix in
+# registers / in LDS
 SHAPES = [(1, 1), (6, 3), (16, 4), (12, 8), (5, 5), (17, 1), (20, 4), (32, 3),
           (13, 6), (24, 8), (31, 9), (32, 16), (4, 12)]
 
@@ -85,6 +86,26 @@ def test_table_codes_at_any_size_and_alignment(pkg, dev, k, m):
     _check(pkg, dev, k, m, n + 2047, lambda j: (5 * j + 3) % 16, lambda i: (7 * i + 1) % 16)
 
 
+@pytest.mark.parametrize("k,m", [(5, 5), (12, 5), (10, 6), (11, 7), (6, 8)])
+def test_any_kernel_with_five_to_eight_outputs(pkg, dev, k, m):
+    """Shards just past 2 MiB, where these codes take any_kernel: no edge, a tail,
+    both edges, and outputs at offsets of their own."""
+    n = 2 << 20
+    _check(pkg, dev, k, m, n + 16, lambda j: 0, lambda i: 0)
+    _check(pkg, dev, k, m, n + 21, lambda j: 0, lambda i: 0)
+    _check(pkg, dev, k, m, n + 33, lambda j: 9, lambda i: 9)
+    _check(pkg, dev, k, m, n + 1029, lambda j: (5 * j + 3) % 16, lambda i: (7 * i + 1) % 16)
+
+
+@pytest.mark.parametrize("k,m,n", [(24, 8, (6 << 20) + 13), (16, 8, (20 << 20) + 13),
+                                   (32, 16, (5 << 20) + 13)])
+def test_wide_kernel_over_several_steps(pkg, dev, k, m, n):
+    """Shards of which every wave of wide_kernel's capped grid codes several
+    steps, loading one while it codes another, with both edges."""
+    _check(pkg, dev, k, m, n, lambda j: (5 * j + 3) % 16, lambda i: (7 * i + 1) % 16)
+    _check(pkg, dev, k, m, n, lambda j: 4, lambda i: 4)
+
+
 @pytest.mark.parametrize("m", [1, 4, 7, 16])
 def test_sums_of_256_ones(pkg, dev, m):
     """32 equal coefficients whose bit matrix has a row of ones: on shards of
@@ -100,6 +121,39 @@ def test_sums_of_256_ones(pkg, dev, m):
     ones[5][700:] = 3   # both kinds of column next to each other
     for co in (coeff, np.full((m, 32), c, np.uint8)):
         _check(pkg, dev, 32, m, n, lambda j: 0, lambda i: 0, coeff=co, data=ones)
+
+
+@pytest.mark.parametrize("m", [1, 7, 16])
+def test_sums_of_256_ones_batched(pkg, dev, m):
+    """The same rows through the batched encode and decode: units of 0xFF, some
+    short, some not there."""
+    c = next(c for c in range(1, 256)
+             if any(all(int(oracle.gf_mul(c, 1 << b)) >> bit & 1 for b in range(8)) for bit in range(8)))
+    C = np.full((m, 32), c, np.uint8)
+    C[: m // 2] = oracle.cauchy(32, m)[: m // 2]
+    k, unit, n = 32, 1040, 5
+    ln = np.full((n, k), unit, np.uint32)
+    ln[1, 3], ln[2, :] = 517, 1039
+    ln[3, 7] = 0
+    units = torch.full((n, k, unit), 0xFF, dtype=torch.uint8, device=dev)
+    ptr = units.data_ptr() + unit * torch.arange(n * k, dtype=torch.int64, device=dev).view(n, k)
+    ptr[3, 7] = 0
+    d_len = torch.from_numpy(ln.view(np.int32)).to(dev)
+    grid = [[np.full(int(ln[s, j]), 0xFF, np.uint8) if ln[s, j] else None for j in range(k)]
+            for s in range(n)]
+    want = oracle.encode_batched(C, grid, ln, unit)
+    lib, stream = pkg._lib, pkg.codec.stream_handle(torch.cuda.current_stream(), dev)
+    out = torch.zeros((2, n, m, unit), dtype=torch.uint8, device=dev)
+    o_ptr = out.data_ptr() + unit * torch.arange(2 * n * m, dtype=torch.int64, device=dev).view(2, n, m)
+    o_len = torch.full((n, m), unit, dtype=torch.int32, device=dev)
+    lib.check(lib.lib().ec_encode_batched(lib.u8ptr(C), k, m, ptr.data_ptr(), d_len.data_ptr(),
+                                          o_ptr[0].data_ptr(), n, unit, stream), "ec_encode_batched")
+    lib.check(lib.lib().ec_decode_batched(lib.u8ptr(C), k, m, ptr.data_ptr(), d_len.data_ptr(),
+                                          o_ptr[1].data_ptr(), o_len.data_ptr(), n, unit, stream),
+              "ec_decode_batched")
+    torch.cuda.synchronize()
+    for got in out:
+        assert np.array_equal(got.cpu().numpy(), want)
 
 
 @pytest.mark.parametrize("k,m", [(6, 3), (10, 6), (24, 8), (20, 4)])
