@@ -60,8 +60,8 @@ int ec_encode_batched(const uint8_t* coeff, int k, int m, const uint64_t* d_data
   if (n_stripes == 0) return EC_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!ec::fast_shape(k, m))
-    return ec::batched_wide(m, coeff, k, d_data_ptrs, d_data_len, nullptr, d_parity_ptrs,
-                                      nullptr, n_stripes, unit_bytes, false, st);
+    return ec::batched_wide(k, m, coeff, d_data_ptrs, d_data_len, d_parity_ptrs, nullptr,
+                            n_stripes, unit_bytes, st);
   return ec::kBatchTable[k - 1][m - 1](coeff, d_data_ptrs, d_data_len, d_parity_ptrs, nullptr,
                                        n_stripes, unit_bytes, st);
 }
@@ -76,8 +76,8 @@ int ec_decode_batched(const uint8_t* rows, int k, int e, const uint64_t* d_surv_
   if (n_stripes == 0) return EC_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!ec::fast_shape(k, e))
-    return ec::batched_wide(e, rows, k, d_surv_ptrs, d_surv_len, nullptr, d_out_ptrs,
-                                      d_out_len, n_stripes, unit_bytes, false, st);
+    return ec::batched_wide(k, e, rows, d_surv_ptrs, d_surv_len, d_out_ptrs, d_out_len, n_stripes,
+                            unit_bytes, st);
   return ec::kBatchTable[k - 1][e - 1](rows, d_surv_ptrs, d_surv_len, d_out_ptrs, d_out_len,
                                        n_stripes, unit_bytes, st);
 }

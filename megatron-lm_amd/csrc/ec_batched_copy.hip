@@ -54,8 +54,8 @@ int ec_encode_batched_copy(const uint8_t* coeff, int k, int m, const uint64_t* d
   // stripes of coefficient 1 (the descriptor arrays read as [n_stripes * k][1]).
   const uint64_t units = (uint64_t)n_stripes * (uint64_t)k;
   if (units > 0xffffffffull) return EC_ERANGE;
-  s = ec::batched_wide(m, coeff, k, d_data_ptrs, d_data_len, nullptr, d_parity_ptrs,
-                                 nullptr, n_stripes, unit_bytes, false, st);
+  s = ec::batched_wide(k, m, coeff, d_data_ptrs, d_data_len, d_parity_ptrs, nullptr, n_stripes,
+                       unit_bytes, st);
   if (s != EC_OK) return s;
   const uint8_t one = 1;
   return ec::batched_fast(1, 1, &one, d_data_ptrs, d_data_len, d_copy_ptrs, nullptr,

@@ -48,14 +48,14 @@ namespace ec {
 
 // Launchers shared between translation units.  batched_fast (ec_batched.hip)
 // runs the fully unrolled batched kernel for k <= 16, m <= 4; batched_wide
-// (ec_update.hip) the run-time-k kernels for any code up to EC_MAX_K x
-// EC_MAX_M, as an encode/decode (update = false) or a parity update.
+// (ec_update.hip) the encode or decode of any other code up to EC_MAX_K x
+// EC_MAX_M, on the matrix cores or on permute tables.
 int batched_fast(int k, int m, const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
                  const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,
                  uint32_t unit_bytes, hipStream_t st);
-int batched_wide(int m, const uint8_t* coeff, int k, const uint64_t* dptr, const uint32_t* dlen,
-                 const uint64_t* optr, const uint64_t* pptr, const uint32_t* olen,
-                 uint32_t n_stripes, uint32_t unit_bytes, bool update, hipStream_t st);
+int batched_wide(int k, int m, const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
+                 const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,
+                 uint32_t unit_bytes, hipStream_t st);
 
 namespace {
 

@@ -632,7 +632,7 @@ int launch_any(const uint8_t* coeff, const uint8_t* const* d, uint8_t* const* o,
     hipLaunchKernelGGL((any_kernel<K, M, false>), dim3(grid), dim3(B), 0, st, a);
   else if constexpr (M <= kFastMaxM)
     hipLaunchKernelGGL((any_kernel<K, M, true>), dim3(grid), dim3(B), 0, st, a);
-  else   // shards past 32 GiB
+  else   // more steps than one grid
     return wide_fn(K, M)(coeff, K, M, d, o, f, st);
   return hip_status();
 }
@@ -736,21 +736,18 @@ template <int... Ks>
 constexpr auto xor_table(std::integer_sequence<int, Ks...>) {
   return std::array<XorFn, sizeof...(Ks)>{&launch_xor<Ks + 1>...};
 }
+template <int K, int M>
+constexpr AnyFn any_entry() {
+  if constexpr (any_reached(K, M)) return &launch_any<K, M>;
+  else return nullptr;
+}
 template <int K, int... Ms>
 constexpr auto any_row(std::integer_sequence<int, Ms...>) {
-  return std::array<AnyFn, sizeof...(Ms)>{&launch_any<K, Ms + 1>...};
-}
-template <int K>
-constexpr auto any_row_of() {
-  constexpr int kMs = K <= kAnyDeepMaxK ? kAnyMaxM : kFastMaxM;
-  std::array<AnyFn, kAnyMaxM> r{};
-  const auto row = any_row<K>(std::make_integer_sequence<int, kMs>{});
-  for (int i = 0; i < kMs; ++i) r[i] = row[i];
-  return r;
+  return std::array<AnyFn, sizeof...(Ms)>{any_entry<K, Ms + 1>()...};
 }
 template <int... Ks>
 constexpr auto any_table(std::integer_sequence<int, Ks...>) {
-  return std::array<std::array<AnyFn, kAnyMaxM>, sizeof...(Ks)>{any_row_of<Ks + 1>()...};
+  return std::array<std::array<AnyFn, kAnyMaxM>, sizeof...(Ks)>{any_row<Ks + 1>(std::make_integer_sequence<int, kAnyMaxM>{})...};
 }
 template <int... Ks>
 constexpr auto any_xor_table(std::integer_sequence<int, Ks...>) {
@@ -758,13 +755,23 @@ constexpr auto any_xor_table(std::integer_sequence<int, Ks...>) {
 }
 using TableFn = int (*)(const uint8_t*, int, const uint8_t* const*, uint8_t* const*, const Frame&,
                         hipStream_t);
+template <int M>
+constexpr TableFn table_entry() {
+  if constexpr (table_reached(M)) return &launch_table<M>;
+  else return nullptr;
+}
 template <int... Ms>
 constexpr auto table_table(std::integer_sequence<int, Ms...>) {
-  return std::array<TableFn, sizeof...(Ms)>{&launch_table<Ms + 1>...};
+  return std::array<TableFn, sizeof...(Ms)>{table_entry<Ms + 1>()...};
+}
+template <int KH, int MH>
+constexpr WideFn wide_entry() {
+  if constexpr (core_reached(KH, MH)) return &launch_wide<KH, MH>;
+  else return nullptr;
 }
 template <int KH, int... Ms>
 constexpr auto wide_row(std::integer_sequence<int, Ms...>) {
-  return std::array<WideFn, sizeof...(Ms)>{&launch_wide<KH, Ms + 1>...};
+  return std::array<WideFn, sizeof...(Ms)>{wide_entry<KH, Ms + 1>()...};
 }
 constexpr int kWideKH = EC_MAX_K / 4, kWideMH = EC_MAX_M / 2;
 template <int... Ks>

@@ -340,13 +340,16 @@ int launch_core(const uint8_t* coeff, int k, int m, const uint64_t* dptr, const 
   return hip_status();
 }
 
-constexpr uint64_t kBatchTableBytes = 16u << 20;   // of each position
-
 using CoreFn = int (*)(const uint8_t*, int, int, const uint64_t*, const uint32_t*,
                        const uint64_t*, const uint32_t*, uint32_t, uint32_t, hipStream_t);
+template <int KH, int MH>
+constexpr CoreFn core_entry() {
+  if constexpr (core_reached(KH, MH)) return &launch_core<KH, MH>;
+  else return nullptr;
+}
 template <int KH, int... Ms>
 constexpr auto core_row(std::integer_sequence<int, Ms...>) {
-  return std::array<CoreFn, sizeof...(Ms)>{&launch_core<KH, Ms + 1>...};
+  return std::array<CoreFn, sizeof...(Ms)>{core_entry<KH, Ms + 1>()...};
 }
 template <int... Ks>
 constexpr auto core_table(std::integer_sequence<int, Ks...>) {
@@ -383,10 +386,11 @@ int update_fast(const uint8_t* coeff, const uint64_t* nptr, const uint64_t* optr
 // optr unused) or the parity update, with B-lane workgroups on B * 16-byte
 // tiles: the encode walks spans of `span` bytes (0: span_bytes()) keeping at
 // least 2048 workgroups, the update one tile per workgroup.
-template <int M, int B>
+// span: bytes of each unit that a workgroup walks (0: span_bytes).
+template <int M, int B, bool UPDATE>
 int launch_batched_wide_b(const uint8_t* coeff, int k, const uint64_t* dptr, const uint32_t* dlen,
                           const uint64_t* optr, const uint64_t* pptr, const uint32_t* olen,
-                          uint32_t n_stripes, uint32_t unit_bytes, bool update, hipStream_t st,
+                          uint32_t n_stripes, uint32_t unit_bytes, hipStream_t st,
                           uint32_t span) {
   BatchWideArgs a;
   a.dptr = dptr;
@@ -400,7 +404,7 @@ int launch_batched_wide_b(const uint8_t* coeff, int k, const uint64_t* dptr, con
   a.tiles_per_unit = (unit_bytes / 16u + B - 1) / B;
   const uint64_t total_tiles = (uint64_t)n_stripes * a.tiles_per_unit;
   uint64_t tpb = 1;
-  if (!update) {
+  if (!UPDATE) {
     tpb = (span ? span : span_bytes(unit_bytes)) / (B * 16u);
     if (tpb < 1) tpb = 1;
     if (total_tiles / tpb < 2048) tpb = total_tiles / 2048;
@@ -414,7 +418,7 @@ int launch_batched_wide_b(const uint8_t* coeff, int k, const uint64_t* dptr, con
   a.by_blocks = make_fastdiv(a.blocks_per_unit);
   const uint64_t blocks = (uint64_t)n_stripes * a.blocks_per_unit;
   if (blocks > 0x7fffffffull) return EC_ERANGE;
-  if (update)
+  if constexpr (UPDATE)
     hipLaunchKernelGGL((update_wide_kernel<M, B>), dim3((unsigned)blocks), dim3(B), 0, st, a);
   else
     hipLaunchKernelGGL((batched_wide_kernel<M, B>), dim3((unsigned)blocks), dim3(B), 0, st, a);
@@ -434,13 +438,19 @@ int launch_batched_wide_b(const uint8_t* coeff, int k, const uint64_t* dptr, con
 // units 4995 -> 4747, RS(24,8) over 1 MiB units 3980 -> 3815).
 template <int M>
 int launch_batched_wide(const uint8_t* coeff, int k, const uint64_t* dptr, const uint32_t* dlen,
-                        const uint64_t* optr, const uint64_t* pptr, const uint32_t* olen,
-                        uint32_t n_stripes, uint32_t unit_bytes, bool update, hipStream_t st) {
-  if (M <= 4 && !update)
-    return launch_batched_wide_b<M, 64>(coeff, k, dptr, dlen, optr, pptr, olen, n_stripes,
-                                        unit_bytes, update, st, 64 * 16);
-  return launch_batched_wide_b<M, kBlock>(coeff, k, dptr, dlen, optr, pptr, olen, n_stripes,
-                                          unit_bytes, update, st, 0);
+                        const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,
+                        uint32_t unit_bytes, hipStream_t st) {
+  constexpr int B = M <= 4 ? 64 : kBlock;
+  return launch_batched_wide_b<M, B, false>(coeff, k, dptr, dlen, nullptr, pptr, olen, n_stripes,
+                                            unit_bytes, st, M <= 4 ? B * 16 : 0);
+}
+
+template <int M>
+int launch_update_wide(const uint8_t* coeff, int k, const uint64_t* nptr, const uint64_t* optr,
+                       const uint32_t* len, const uint64_t* pptr, uint32_t n_stripes,
+                       uint32_t unit_bytes, hipStream_t st) {
+  return launch_batched_wide_b<M, kBlock, true>(coeff, k, nptr, len, optr, pptr, nullptr,
+                                                n_stripes, unit_bytes, st, 0);
 }
 
 using UpdFn = int (*)(const uint8_t*, const uint64_t*, const uint64_t*, const uint32_t*,
@@ -457,33 +467,35 @@ constexpr auto upd_table(std::integer_sequence<int, Ks...>) {
 }
 const auto kUpdTable = upd_table(std::make_integer_sequence<int, kFastMaxK>{});
 using BatchWideFn = int (*)(const uint8_t*, int, const uint64_t*, const uint32_t*,
-                            const uint64_t*, const uint64_t*, const uint32_t*, uint32_t, uint32_t,
-                            bool, hipStream_t);
+                            const uint64_t*, const uint32_t*, uint32_t, uint32_t, hipStream_t);
+template <int M>
+constexpr BatchWideFn batch_wide_entry() {
+  if constexpr (batch_table_reached(M)) return &launch_batched_wide<M>;
+  else return nullptr;
+}
+using UpdWideFn = int (*)(const uint8_t*, int, const uint64_t*, const uint64_t*, const uint32_t*,
+                          const uint64_t*, uint32_t, uint32_t, hipStream_t);
 template <int... Ms>
 constexpr auto batch_wide_table(std::integer_sequence<int, Ms...>) {
-  return std::array<BatchWideFn, sizeof...(Ms)>{&launch_batched_wide<Ms + 1>...};
+  return std::array<BatchWideFn, sizeof...(Ms)>{batch_wide_entry<Ms + 1>()...};
+}
+template <int... Ms>
+constexpr auto upd_wide_table(std::integer_sequence<int, Ms...>) {
+  return std::array<UpdWideFn, sizeof...(Ms)>{&launch_update_wide<Ms + 1>...};
 }
 const auto kBatchWideTable = batch_wide_table(std::make_integer_sequence<int, EC_MAX_M>{});
-
+const auto kUpdWideTable = upd_wide_table(std::make_integer_sequence<int, EC_MAX_M>{});
 
 }  // namespace
 
-int batched_wide(int m, const uint8_t* coeff, int k, const uint64_t* dptr, const uint32_t* dlen,
-                 const uint64_t* optr, const uint64_t* pptr, const uint32_t* olen,
-                 uint32_t n_stripes, uint32_t unit_bytes, bool update, hipStream_t st) {
-  if (m < 1 || m > EC_MAX_M || k < 1 || k > EC_MAX_K) return EC_ERANGE;
-  // The tables where they clearly cost less (table_cost against core_cost, see
-  // ec_mfma.h) and enough stripes run to be bound by it (us, tables / matrix
-  // cores, 100 tensors in 64 KiB units: RS(10,6) 293 / 316, RS(20,2) 176 / 192;
-  // RS(6,8) 406 / 394, RS(20,4) 216 / 208, RS(24,8) 341 / 243, RS(32,16) 588 /
-  // 390; RS(10,6) over 5 MB of 16 KiB stripes 25.0 / 21.2).
-  const bool tables = (uint64_t)n_stripes * unit_bytes > kBatchTableBytes &&
-                      4 * table_cost(k, m) <= 3 * core_cost(k, m);
-  if (!update && !tables)
-    return kCoreTable[(k - 1) / 4][(m - 1) / 2](coeff, k, m, dptr, dlen, pptr, olen, n_stripes,
-                                                unit_bytes, st);
-  return kBatchWideTable[m - 1](coeff, k, dptr, dlen, optr, pptr, olen, n_stripes, unit_bytes,
-                                update, st);
+int batched_wide(int k, int m, const uint8_t* coeff, const uint64_t* dptr, const uint32_t* dlen,
+                 const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,
+                 uint32_t unit_bytes, hipStream_t st) {
+  if (m < 1 || m > EC_MAX_M || k < 1 || k > EC_MAX_K || fast_shape(k, m)) return EC_ERANGE;
+  if (batch_tables(k, m, (uint64_t)n_stripes * unit_bytes))
+    return kBatchWideTable[m - 1](coeff, k, dptr, dlen, pptr, olen, n_stripes, unit_bytes, st);
+  return kCoreTable[(k - 1) / 4][(m - 1) / 2](coeff, k, m, dptr, dlen, pptr, olen, n_stripes,
+                                              unit_bytes, st);
 }
 
 }  // namespace ec
@@ -500,8 +512,8 @@ int ec_parity_update(const uint8_t* coeff, int k, int m, const uint64_t* d_new_p
   if (n_stripes == 0) return EC_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!ec::fast_shape(k, m))
-    return ec::kBatchWideTable[m - 1](coeff, k, d_new_ptrs, d_len, d_old_ptrs, d_parity_ptrs,
-                                      nullptr, n_stripes, unit_bytes, true, st);
+    return ec::kUpdWideTable[m - 1](coeff, k, d_new_ptrs, d_old_ptrs, d_len, d_parity_ptrs,
+                                    n_stripes, unit_bytes, st);
   return ec::kUpdTable[k - 1][m - 1](coeff, d_new_ptrs, d_old_ptrs, d_len, d_parity_ptrs,
                                      n_stripes, unit_bytes, st);
 }

@@ -81,6 +81,38 @@ constexpr FlatRoute flat_route(int k, int m, uint64_t nbytes, bool aligned) {
   return table_kernel_pays(k, m, nbytes) ? FlatRoute::kTable : FlatRoute::kWide;
 }
 
+// Whether the batched encode or decode of a code past the unrolled kernels runs
+// on permute tables: where they clearly cost less and enough stripes run to be
+// bound by it (us, tables / matrix cores, 100 tensors in 64 KiB units: RS(10,6)
+// 293 / 316, RS(20,2) 176 / 192; RS(6,8) 406 / 394, RS(20,4) 216 / 208, RS(24,8)
+// 341 / 243, RS(32,16) 588 / 390; RS(10,6) over 5 MB of 16 KiB stripes 25.0 /
+// 21.2).  position_bytes: the bytes of each position, all stripes together.
+constexpr bool batch_tables_pay(int k, int m) {
+  return !fast_shape(k, m) && 4 * table_cost(k, m) <= 3 * core_cost(k, m);
+}
+constexpr uint64_t kBatchTableBytes = 16u << 20;
+constexpr bool batch_tables(int k, int m, uint64_t position_bytes) {
+  return batch_tables_pay(k, m) && position_bytes > kBatchTableBytes;
+}
+
+// Which kernels some call reaches: the only ones that are instantiated.  Those
+// of the matrix cores are shared by the codes with the same kh = ceil(k / 4) and
+// mh = ceil(m / 2).
+constexpr bool any_reached(int k, int m) {
+  return fast_shape(k, m) || (any_shape(k, m) && table_pays(k, m));
+}
+constexpr bool table_reached(int m) {
+  for (int k = 1; k <= EC_MAX_K; ++k)
+    if (flat_route(k, m, UINT64_MAX, true) == FlatRoute::kTable) return true;
+  return false;
+}
+constexpr bool core_reached(int kh, int mh) { return !fast_shape(4 * kh, 2 * mh); }
+constexpr bool batch_table_reached(int m) {
+  for (int k = 1; k <= EC_MAX_K; ++k)
+    if (batch_tables_pay(k, m)) return true;
+  return false;
+}
+
 // Workgroups of one launch at most; more work loops in the kernel.  HIP refuses
 // a grid of 2^32 lanes and more.
 constexpr uint64_t max_grid(uint64_t lanes) {

@@ -26,6 +26,13 @@ int main() {
         else ok = odd == FlatRoute::kWide;
         // single losses of wide codes and XOR of many shards: tables at any size past the small ones
         if (m == 1 && k > ec::kFastMaxK && n > two) ok = ok && odd == FlatRoute::kTable;
+        // a kernel for every route (past any_kernel's one grid its codes go to the matrix cores)
+        if (odd == FlatRoute::kAny) ok = ok && ec::any_reached(k, m);
+        if (odd == FlatRoute::kTable) ok = ok && ec::table_reached(m);
+        if (odd == FlatRoute::kWide || (odd == FlatRoute::kAny && m > ec::kFastMaxM))
+          ok = ok && ec::core_reached((k - 1) / 4 + 1, (m - 1) / 2 + 1);
+        if (ec::batch_tables(k, m, n)) ok = ok && n > ec::kBatchTableBytes && ec::batch_table_reached(m);
+        else if (!ec::fast_shape(k, m)) ok = ok && ec::core_reached((k - 1) / 4 + 1, (m - 1) / 2 + 1);
         if (!ok) {
           std::printf("RS(%d,%d) over %llu bytes: route %d, aligned %d\n", k, m,
                       (unsigned long long)n, (int)odd, (int)even);
