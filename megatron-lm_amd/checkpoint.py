@@ -200,10 +200,10 @@ class GpuSliceCodec:
     fits (see ``snapshot``) and stages it with ``ec_stage_stripes_to_host``;
     otherwise the work goes in chunks of stripes of at most ``chunk_bytes``,
     double-buffered on the device and in pinned host memory: 2 * chunk_bytes
-    of extra HBM and at most 128 MiB of page-locked memory (``_pinned_bytes``).  ``decode`` likewise takes one
-    (k, stripes, unit_bytes) block when it fits, else chunks, and moves the
-    slices up with ``ec_stage_to_device`` through at most 512 MiB of page-locked
-    memory (``_pinned_load_bytes``).
+    of extra HBM and about 128 MiB of page-locked memory (``_pinned_bytes``).
+    ``decode`` likewise takes one (k, stripes, unit_bytes) block when it fits,
+    else chunks, and moves the slices up with ``ec_stage_to_device`` through
+    about 512 MiB of page-locked memory at most (``_pinned_load_bytes``).
 
     The slices own their host array (they are views of it): the codec keeps
     no reference to an array it handed out, so nothing the caller holds,
@@ -294,22 +294,23 @@ class GpuSliceCodec:
 
     def _pinned_bytes(self, total: int) -> int:
         """Bytes of pinned memory to stage a block of ``total`` bytes down
-        through, two halves: a half is a 32nd of the total, between 16 and
-        64 MiB, within 2 * ``chunk_bytes`` in all.  The first half's transfer
-        and the last one's host copy overlap nothing, so halves of 1 GiB left
-        a block of 1.07 GB with two steps one after the other: saving a 0.80 GB
-        state (RS(12,4), 64 KiB units) took 32.0 ms with them, 21.0 with these;
-        the link alone takes about 19.  A half goes down in one transfer, but
-        its copying threads are started for it, about as long as 4 MiB take on
-        the link.  Measured on MI355X (RS(12,4), ms a save, in one piece /
-        halves of 4, 8, 16, 32 and 64 MiB):
-           10 MiB  0.71 / 0.71  0.74
-           20 MiB  1.19 / 1.29  1.10  1.05
-           50 MiB  2.34 / 2.35  1.80  1.87  2.03  2.38
-          200 MiB  8.64 / 9.27  6.40  6.06  6.15  6.45
-         1000 MiB  33.2 / 42.0  29.2  27.2  26.9  27.2"""
-        half = max(16 << 20, min(64 << 20, total // 32))
-        return min(2 * self.chunk_bytes, 2 * total, 2 * half)
+        through, two halves, within 2 * ``chunk_bytes`` in all.  The first
+        half's transfer and the last one's host copy overlap nothing, so a block
+        goes in several pieces; but a half's copying threads are started for
+        it, about as long as 4 MiB take on the link, so pieces are 12 to 16 MiB,
+        a 32nd of the block from 512 MiB on, up to about 64 MiB, and equal (a
+        short last one costs as much).  Measured on MI355X, ms a save of these
+        blocks (RS(20,4) and RS(12,4)):
+          18 MiB   in one 1.03, two 0.86, 16 + 2 1.10
+          24 MiB   in one 1.09, two 0.95, three 0.92, 16 + 8 0.96
+          34 MiB   in one 1.39, two 1.22, three 1.22, 16 + 16 + 2 1.31
+         266 MiB   in one 8.64, by 8 MiB 6.40, 16 6.06, 32 6.15, 64 6.45
+        1333 MiB   by 1 GiB 33.2, 8 MiB 29.2, 16 27.2, 32 26.9, 64 27.2 (the
+                   link alone takes about 25)"""
+        MiB = 1 << 20
+        piece = max(12 * MiB, min(16 * MiB, total // 4), min(64 * MiB, total // 32))
+        half = -(-total // max(1, (total + piece // 2) // piece))
+        return min(2 * self.chunk_bytes, 2 * (-(-half // 4096) * 4096))
 
     def _pinned_load_bytes(self, row: int, rows: int) -> int:
         """Bytes of pinned memory to stage ``rows`` rows of ``row`` bytes up

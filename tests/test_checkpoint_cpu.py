@@ -181,17 +181,21 @@ def test_load_halves_carry_whole_loads_or_megabytes_per_row(pkg, k):
     assert small._pinned_load_bytes(1 << 30, k) == 2 << 20
 
 
-def test_save_halves_carry_small_saves_whole():
-    """A half of the download's pinned memory costs a set of host threads: a
-    block of up to 16 MiB goes down in one, larger ones in halves of 16 to 64."""
+def test_save_halves_are_few_and_equal():
+    """A half of the download's pinned memory costs a set of host threads: small
+    blocks go down in one, larger ones in equal pieces of 9 to about 64 MiB."""
     import __graft_entry__
     __graft_entry__.load_package()
     from megatron_lm_amd.checkpoint import GpuSliceCodec
     codec = GpuSliceCodec(12, 4, 65536)
-    for total in (65536, 5 << 20, 16 << 20):
-        assert codec._pinned_bytes(total) == 2 * total
-    for total in (20 << 20, 100 << 20, 1 << 30, 20 << 30):
-        assert 16 << 20 <= codec._pinned_bytes(total) // 2 <= 64 << 20
+    for total in (65536, 4096 * 5 + 16, 5 << 20, 16 << 20):
+        assert codec._pinned_bytes(total) // 2 == -(-total // 4096) * 4096
+    for total in [m << 20 for m in (18, 20, 24, 31, 34, 55, 100, 266, 1000, 1333, 20_000)] + [10**9 + 48]:
+        half = codec._pinned_bytes(total) // 2
+        assert 9 << 20 <= half <= 66 << 20
+        tail = total % half
+        assert tail == 0 or tail > half * 7 // 8, f"{total}: pieces of {half} leave {tail}"
+    assert GpuSliceCodec(12, 4, 4096, chunk_bytes=1 << 20)._pinned_bytes(1 << 30) == 2 << 20
 
 
 def test_slice_host_arrays_are_reused_only_after_release():
