@@ -109,10 +109,11 @@ int ec_decode_matrix(const uint8_t* coeff, int k, int m, const int* erased,
 /* XOR parity: d_parity[b] = XOR_{j<k} d_data[j][b].  d_data is a host array
  * of k device pointers.  Any size and any alignment of each shard, in one
  * kernel launch; shards of whole 16-byte chunks at 16-byte-aligned addresses
- * run fastest.  The same holds for ec_rs_encode and ec_rs_decode.  nbytes = 0 returns
- * EC_OK without touching the shard pointers (empty tensors may have null
- * addresses); so do those two.  Serves manager.save at
- * checkpointing.py:538-541 for m = 1. */
+ * run fastest.  An output may lie exactly over an input (the same address):
+ * each byte depends on its own column only.  The same holds for ec_rs_encode
+ * and ec_rs_decode.  nbytes = 0 returns EC_OK without touching the shard
+ * pointers (empty tensors may have null addresses); so do those two.  Serves
+ * manager.save at checkpointing.py:538-541 for m = 1. */
 int ec_xor_encode(const uint8_t* const* d_data, int k, uint8_t* d_parity,
                   uint64_t nbytes, ec_stream_t stream);
 
@@ -141,13 +142,14 @@ int ec_rs_decode(const uint8_t* rows, int k, int e,
  * The arrays are dense: the kernels read every entry of a stripe, also the
  * length of an absent unit (ignored).
  * unit_bytes must be a multiple of 16 (EC_EALIGN otherwise) and at most
- * 2 GiB (EC_ERANGE).  Units and
- * parity units at 16-byte-aligned addresses take the vector path; others are
- * read and written byte by byte, and no byte past a unit's valid length is
- * read.  Units of 4 KiB and up stream at HBM rate; smaller units work but
- * run a slower byte-granular path.  k <= EC_MAX_K and m <= EC_MAX_M
- * (EC_ERANGE otherwise); k <= 16, m <= 4 run fully unrolled kernels, wider
- * codes a kernel with k at run time.  The units come from the ragged
+ * 2 GiB (EC_ERANGE).  Units and parity units may lie at any address; those
+ * at 16-byte-aligned ones run fastest (fp32 views of one flat buffer take
+ * up to 20 % longer).  No byte past a unit's valid length is read, and an output's
+ * last partial 16 bytes are stored byte by byte.  Units of 1 KiB and up
+ * stream at HBM rate (a workgroup takes at most one unit's 1 KiB, so smaller
+ * ones leave lanes idle).  k <= EC_MAX_K and m <= EC_MAX_M (EC_ERANGE
+ * otherwise); k <= 16, m <= 4 run fully unrolled kernels, wider codes the
+ * matrix cores or permute tables with k at run time.  The units come from the ragged
  * shard list of tensor_aware_state_dict.py:179-184 (MCoreTensorAwareStateDict
  * .tensors), chunked in order. */
 int ec_encode_batched(const uint8_t* coeff, int k, int m,
@@ -161,8 +163,8 @@ int ec_encode_batched(const uint8_t* coeff, int k, int m,
  * copy, so coding a checkpoint into one contiguous block (the data units as
  * the block's first k rows, the parity as its last m) costs one pass over
  * HBM.  Copies must not overlap the inputs or the parity.  Same limits and
- * alignment rules as ec_encode_batched (16-byte aligned copies take the fast
- * path); k > 16 or m > 4 runs the encode and the copies as two launches.
+ * alignment rules as ec_encode_batched (16-byte aligned copies run
+ * fastest); k > 16 or m > 4 runs the encode and the copies as two launches.
  * Serves manager.save at checkpointing.py:538-541: the snapshot of the
  * tensors of tensor_aware_state_dict.py:179-184 that training may overwrite
  * as soon as the call's work has run. */

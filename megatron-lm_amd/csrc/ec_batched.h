@@ -62,9 +62,11 @@ constexpr bool early_tables() {
 
 // Two outputs of eight to ten units run fastest with three waves per SIMD:
 // RS(8,2) 336 us against 345 with the four that its registers allow, RS(10,2)
-// 333 against 375 with the two that it takes by itself.  Codes with more
-// outputs keep theirs (RS(12,4) with three 1392 against 1328, RS(6,3) 606 /
-// 587, RS(10,4) 403 / 383; five spill).
+// 333 against 375 with the two that it takes by itself, RS(9,2) in 64 KiB /
+// 1 MiB units 213 / 233 against 219 / 240.  The others keep what the compiler
+// gives them: RS(12,4) four waves (1328 us, with three 1392), RS(10,4) four (383 /
+// 403), RS(6,3) three (144 registers; 258 us in 64 KiB and 286 in 1 MiB units,
+// forced to four 273 and 310).
 template <int K, int M, bool COPY>
 constexpr bool three_waves() {
   return early_tables<K, M, COPY>() && M == 2;

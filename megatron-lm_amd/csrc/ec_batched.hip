@@ -1,7 +1,7 @@
 // ec_batched.hip — ec_encode_batched and ec_decode_batched: one launch over
 // the stripes of a ragged unit layout, k <= 16 and m <= 4 through the fully
-// unrolled batched_kernel (ec_batched.h), wider codes through
-// batched_wide_kernel (ec_update.hip).
+// unrolled batched_kernel (ec_batched.h), wider codes through batched_wide
+// (ec_update.hip).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

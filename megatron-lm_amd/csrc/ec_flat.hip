@@ -428,7 +428,9 @@ __global__ void __launch_bounds__(kTableBlock) table_kernel(const TableArgs a) {
 // permute tables first): RS(24,8) over 32 MiB shards 4.08 -> 5.38 (one step
 // per wave without the loads ahead 5.19), RS(32,16) 2.69 -> 3.93 (3.10),
 // RS(20,12) 3.57 -> 4.27 (3.80), RS(16,8) over 64 MiB 4.47 -> 5.61 (5.16).
-// With the MFMAs taken out the same kernel moves 5.7-6.0.
+// With the MFMAs taken out the same kernel moves 5.7-6.0.  By counters the
+// matrix cores work 42 % of the time and the vector ALUs 40 % (RS(24,8));
+// RS(32,16) 66 and 40.
 //   m <= 4 (wide_narrow_kernel): memory-bound, one step per wave and none
 // ahead: RS(20,4) over 64 MiB 5.70 -> 6.12 (with loads ahead 5.6), RS(24,4)
 // 5.62 -> 5.90.

@@ -42,12 +42,13 @@ struct UpdateArgs {
 // parity loads of all U chunks are issued first (they do not depend on the
 // delta), then each changed unit's new and old chunks, so a lane has
 // U * (M + 2) loads in flight.  Misaligned units (views at arbitrary
-// offsets) are realigned there (load_realign); the aligned case keeps plain
-// loads (realigning every load cost the 1 % update 5 %).  The parity
+// offsets) are read there with unaligned loads (load_realign); the aligned case
+// keeps plain ones (load_realign throughout cost the 1 % update 5 %).  The parity
 // stores are nt+sc1 buffer stores on the tile's wave-uniform base
 // (store_wave): config 5's 1 % update 310.9 -> 304.9 us against global nt
 // stores, same box; buffer loads as well measured 312.6.  Any other tile
-// takes the byte-granular path one chunk at a time.  Parity chunks that
+// takes its changed units in pairs, at clamped unaligned addresses with a
+// unit's last chunk shifted into place (clip_chunk).  Parity chunks that
 // start at or past the end of the stripe's longest changed unit are neither
 // read nor written: the delta is zero there.
 template <int K, int M, int B, int U>

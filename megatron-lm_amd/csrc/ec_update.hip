@@ -2,8 +2,8 @@
 // k <= 16, m <= 4) and the batched kernels for wide codes
 // (batched_core_kernel on the matrix cores; batched_wide_kernel and
 // update_wide_kernel on permute tables, k at run time; up to
-// EC_MAX_K x EC_MAX_M), which ec_batched.hip and ec_batched_copy.hip reach
-// through batched_wide().
+// EC_MAX_K x EC_MAX_M).  ec_batched.hip and ec_batched_copy.hip reach the first
+// two through batched_wide(), ec_parity_update the third.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -22,8 +22,11 @@ namespace {
 // instantiated fast path (k > 16 or m > 4): k at run time, M a template
 // parameter, one 16-byte chunk per lane (4 KiB tiles).  A workgroup stages
 // its stripe's descriptors and the m x k tables in LDS; fast tiles issue the
-// unit loads in groups of kWideGroup, edge tiles take the units one at a
-// time with byte-granular ends, as in the fixed-size kernels.
+// unit loads in groups of kWideGroup; tiles with unit ends or misaligned
+// addresses take the units one at a time, with one unaligned load each at a
+// clamped address (load_clip).  On views of one flat buffer that is as fast as
+// the aligned tiles (300 tensors in 64 KiB units, us, aligned / views: RS(10,6)
+// 398 / 388, RS(17,1) 241 / 223): enough waves run to hide the single load.
 
 struct BatchWideArgs {
   const uint64_t* dptr;  // [n_stripes][k] (update: new units, 0 = unchanged)
@@ -429,13 +432,12 @@ int launch_batched_wide_b(const uint8_t* coeff, int k, const uint64_t* dptr, con
 // tile each, like the fixed-size batched kernel; wider outputs and the update
 // keep 256-lane workgroups.  Both keep launch order for every unit size:
 // the fixed-size kernel's 8 slices for large units (SpanGrid) gained nothing
-// here and cost RS(16,6) over 4 MiB units 11 % (encode 0.606 -> 0.539 of the
-// roofline; RS(20,4) 4 MiB 0.661 -> 0.659, RS(24,8) 2 MiB 0.498 -> 0.496;
-// the 1 % update of RS(12,4) and RS(8,2) over 4 MiB units within 1 %).  Measured on MI355X (HBM traffic, GB/s, 8 GiB
-// buffers): RS(20,4) over 4 MiB units encode 5041 -> 5314, decode of 4
-// positions 4886 -> 5136; with m >= 6 the per-workgroup table build (m * k
-// tables) made one-wavefront workgroups 5 % slower (RS(16,6) over 64 KiB
-// units 4995 -> 4747, RS(24,8) over 1 MiB units 3980 -> 3815).
+// here and cost up to 11 %.  Measured on MI355X when all wide codes ran on these
+// tables (HBM traffic, GB/s, 8 GiB buffers; of these codes only decodes of one
+// to three positions still do): one wavefront against 256 lanes with m = 4,
+// RS(20,4) over 4 MiB units, encode 5041 -> 5314, decode 4886 -> 5136; with
+// m >= 6 the per-workgroup table build (m * k tables) made one-wavefront
+// workgroups 5 % slower (RS(16,6) over 64 KiB units 4995 -> 4747).
 template <int M>
 int launch_batched_wide(const uint8_t* coeff, int k, const uint64_t* dptr, const uint32_t* dlen,
                         const uint64_t* pptr, const uint32_t* olen, uint32_t n_stripes,

@@ -123,7 +123,8 @@ def test_gpu_incremental_saves_equal_full_encodes(pkg, dev, k, m, unit):
 
 def test_gpu_incremental_saves_over_misaligned_views(pkg, dev):
     """Tensors that are views of one flat buffer at odd byte offsets (the
-    update and the unit copy take their realigning and byte-granular paths):
+    update and the unit copy take their paths for unaligned addresses and unit
+    ends):
     incremental saves equal the oracle codec's full encodes, with the bytes
     between the views left alone."""
     from megatron_lm_amd.checkpoint import GpuSliceCodec

@@ -105,7 +105,7 @@ def test_rs_encode_wide_codes(pkg, dev, k, m, offset):
 
 
 def test_rs_encode_generic_kernel_mixed_misalignment(pkg, dev):
-    """Different misalignments take the byte path throughout, wide codes too."""
+    """Every shard at a misalignment of its own, a wide code."""
     k, m, n = 20, 6, 9999
     rng = np.random.default_rng(5)
     d = _host(rng, k, n)
@@ -676,8 +676,8 @@ def test_zero_byte_inputs(pkg, dev):
 @pytest.mark.parametrize("n", [5, 31, 4096 + 7, 100_003])
 @pytest.mark.parametrize("k,m", [(6, 3), (4, 1), (20, 6)])
 def test_rs_encode_realigned_inputs(pkg, dev, k, m, n):
-    """Inputs at every misalignment 0..15 with aligned outputs: the wide
-    kernel's realigning loads (two aligned loads + v_alignbyte per shard)."""
+    """Inputs at every misalignment 0..15 with aligned outputs: unaligned
+    16-byte loads."""
     rng = np.random.default_rng(n + 31 * k)
     d = _host(rng, k, n)
     dd = [_to_dev([a], dev, j % 16)[0] for j, a in enumerate(d)]
@@ -1277,9 +1277,9 @@ def test_batched_random_layouts(pkg, dev, seed):
 @pytest.mark.parametrize("seed", range(48))
 def test_flat_random_shards(pkg, dev, seed):
     """Seeded random flat-shard calls: codes from RS(1,1) to RS(24,8) and
-    XOR, sizes from 1 byte to ~300 KiB (vector body and byte tail), each
+    XOR, sizes from 1 byte to ~300 KiB (whole chunks and edges), each
     shard and output at its own offset 0..15 (aligned, one shared
-    misalignment, or mixed: the realigning and the byte kernels), with random
+    misalignment, or mixed), with random
     coefficient matrices as well as the Cauchy block; the encode against the
     oracle and a reconstruction of a random erasure set."""
     r = np.random.default_rng(1000 + seed)
