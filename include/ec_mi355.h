@@ -143,13 +143,13 @@ int ec_rs_decode(const uint8_t* rows, int k, int e,
  * length of an absent unit (ignored).
  * unit_bytes must be a multiple of 16 (EC_EALIGN otherwise) and at most
  * 2 GiB (EC_ERANGE).  Units and parity units may lie at any address; those
- * at 16-byte-aligned ones run fastest (fp32 views of one flat buffer take
- * up to 20 % longer).  No byte past a unit's valid length is read, and an output's
- * last partial 16 bytes are stored byte by byte.  Units of 1 KiB and up
- * stream at HBM rate (a workgroup takes at most one unit's 1 KiB, so smaller
- * ones leave lanes idle).  k <= EC_MAX_K and m <= EC_MAX_M (EC_ERANGE
- * otherwise); k <= 16, m <= 4 run fully unrolled kernels, wider codes the
- * matrix cores or permute tables with k at run time.  The units come from the ragged
+ * at 16-byte-aligned ones run fastest (others at 67 to 98 % of the rate).
+ * No byte past a unit's valid length is read, and an output's last partial
+ * 16 bytes are stored byte by byte.  Units of 1 KiB and up stream at HBM rate
+ * (a workgroup takes at most one unit's 1 KiB, so smaller ones leave lanes
+ * idle).  k <= EC_MAX_K and m <= EC_MAX_M (EC_ERANGE otherwise); k <= 16,
+ * m <= 4 run fully unrolled kernels, wider codes the matrix cores or permute
+ * tables with k at run time.  The units come from the ragged
  * shard list of tensor_aware_state_dict.py:179-184 (MCoreTensorAwareStateDict
  * .tensors), chunked in order. */
 int ec_encode_batched(const uint8_t* coeff, int k, int m,
